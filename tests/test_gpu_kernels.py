@@ -113,6 +113,70 @@ def test_weight_quant_bit_exact():
     assert np.array_equal(host(q8), q8r) and np.array_equal(host(s8), s8r)
 
 
+@pytest.mark.parametrize("n,skew", [(32, 0), (1024, 0), (2048 + 32, 0), (3 * 2048 - 32, 0),
+                                    (32, 1), (2048 + 96, 1)])
+def test_act_quant_edges_and_unaligned(n, skew):
+    """The four-values-per-lane kernels at the edges of their 2048-value
+    workgroups, and the one-value kernels that unaligned operands (skew floats
+    and bytes off) take: bit-exact."""
+    rng = np.random.default_rng(103 + n)
+    x = _wide_range_acts(rng, max(n, 128))[:n].copy()
+    q_ref, s_ref = O.fp8_act_emit(x)
+    raw, off = n // 32, (n // 32 + 15) // 16 * 16
+    announce("act quant n=%d skew=%d" % (n, skew))
+    dx = torch.empty(n + skew, device=DEV)[skew:]
+    dx.copy_(dev(x))
+    q = torch.full((n + skew + 4,), 0xA5, dtype=torch.uint8, device=DEV)
+    s = torch.zeros(off + raw, dtype=torch.uint8, device=DEV)
+    L.emit8_packed(dx, q[skew:], s, n)
+    sh, qh = host(s), host(q)
+    assert np.array_equal(qh[skew:skew + n], q_ref) and (qh[skew + n:] == 0xA5).all()
+    assert np.array_equal(sh[:raw], s_ref) and np.array_equal(sh[off:], s_ref)
+    L.snap8(dx, n)
+    got, want = host(dx), O.fp8_snap(x)
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
+    if n % 128 == 0:
+        m, k = 1, n
+        y = rng.standard_normal((m, k)).astype(np.float32)
+        dx.copy_(dev(y.ravel()))
+        aq_ref, as_ref = O.act_quant_f32s(y, 128)
+        sf = torch.empty(k // 128, device=DEV)
+        L.act_quant_f32s(dx, q[skew:], sf, m, k)
+        assert np.array_equal(host(q)[skew:skew + n], aq_ref.ravel())
+        assert np.array_equal(host(sf).view(np.uint32), as_ref.view(np.uint32).ravel())
+
+
+@pytest.mark.parametrize("rows,cols,skew", [(1, 32, 0), (33, 160, 0), (31, 96, 0), (64, 384, 0),
+                                            (33, 160, 1)])
+def test_weight_quant_edges_and_unaligned(rows, cols, skew):
+    """The vectorised weight encoders at ragged rows and columns, with FP4
+    values on and beside every rounding threshold, and the fallback for
+    unaligned operands: bit-exact."""
+    rng = np.random.default_rng(104 + rows + cols)
+    w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
+    edges = np.array([0.25, 0.75, 1.0, 1.25, 1.75, 2.5, 3.5, 5.0, 6.0], np.float32)
+    edges = np.concatenate([edges, np.nextafter(edges, np.float32(0)),
+                            np.nextafter(edges[:-1], np.float32(9)), [0.0, -0.0, 1e-40]])
+    edges = np.concatenate([edges, edges[:3]]).astype(np.float32)   # largest 6: scale 1
+    w[0, :32] = np.where(rng.random(32) < 0.5, -edges, edges)
+    w[rows - 1, cols - 32:] = np.float32(1e30) if rows > 1 else w[rows - 1, cols - 32:]
+    announce("weight_quant edges %dx%d skew=%d" % (rows, cols, skew))
+    dw = torch.empty(rows * cols + skew, device=DEV)[skew:]
+    dw.copy_(dev(w.ravel()))
+    q4 = torch.empty(rows * cols // 2 + skew, dtype=torch.uint8, device=DEV)[skew:]
+    s4 = torch.empty(rows * cols // 32, dtype=torch.uint8, device=DEV)
+    L.weight_quant_fp4(dw, q4, s4, rows, cols)
+    q4r, s4r = O.weight_quant_fp4(w)
+    assert np.array_equal(host(q4), q4r.ravel()) and np.array_equal(host(s4), s4r.ravel())
+    q8 = torch.empty(rows * cols + skew, dtype=torch.uint8, device=DEV)[skew:]
+    s8 = torch.empty((rows + 31) // 32 * (cols // 32), dtype=torch.uint8, device=DEV)
+    L.weight_quant_fp8(dw, q8, s8, rows, cols)
+    q8r, s8r = O.weight_quant_fp8(w)
+    assert np.array_equal(host(q8), q8r.ravel()) and np.array_equal(host(s8), s8r.ravel())
+
+
 def _quantised_case(rng, m, n, k, fp4):
     x = activations(rng, m, k)
     aq, as_ = O.fp8_act_emit(x)

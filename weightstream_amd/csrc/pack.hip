@@ -6,28 +6,47 @@
 
 namespace ws {
 
-// one thread per 16-byte chunk (row r, K [32c, 32c+32)) and its scale byte
+// One wave per 16-row band and 8-step scale group: lane l (row l % 16, chunks
+// 4 ks + l / 16) copies its eight 16-byte chunks, so the wave reads 64-byte
+// row pieces and writes 8 KB in one run, and stores its eight scale bytes (127
+// past the last step, so the packed buffer is deterministic) as one word
+// pair. One 16-byte chunk per thread in row order scattered the stores:
+// 188.7 M weights 77.6 -> 45 us.
 __global__ __launch_bounds__(256) void prepack_fp4_kernel(const uint8_t *__restrict__ w,
                                                           const uint8_t *__restrict__ s,
                                                           uint8_t *__restrict__ pw,
-                                                          uint8_t *__restrict__ ps, int64_t rows,
+                                                          uint8_t *__restrict__ ps, int64_t groups,
                                                           int cols) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int cpr = cols / 32;  // 32-value chunks per row
-    if (i >= rows * cpr) return;
-    const int64_t r = i / cpr;
-    const int c = (int)(i % cpr);
-    const int ks = c / 4, g = c % 4, ksn = cols / 128, ks8 = (ksn + 7) / 8;
-    const int64_t rt = r / 16;
-    const int lane = (int)(r % 16) + 16 * g;
-    const uint4 v = *(const uint4 *)(w + r * (cols / 2) + (int64_t)c * 16);
-    *(uint4 *)(pw + ((rt * ksn + ks) * 64 + lane) * 16) = v;
-    ps[((rt * ks8 + ks / 8) * 64 + lane) * 8 + ks % 8] = s[r * cpr + c];
-}
-
-__global__ __launch_bounds__(256) void fill_u8_kernel(uint8_t *p, int64_t n, uint8_t v) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = v;
+    const int64_t gi = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);  // band * ks8 + group
+    if (gi >= groups) return;
+    const int lane = threadIdx.x & 63;
+    const int cpr = cols / 32, ksn = cols / 128, ks8 = (ksn + 7) / 8;
+    const int64_t rt = gi / ks8;
+    const int k0 = (int)(gi % ks8) * 8;
+    const int64_t r = rt * 16 + (lane & 15);
+    const uint8_t *src = w + r * (cols / 2), *sc = s + r * cpr;
+    uint4 v[8];
+    uint32_t b[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const int c = 4 * min(k0 + u, ksn - 1) + (lane >> 4);
+        v[u] = *(const uint4 *)(src + (int64_t)c * 16);
+        b[u] = sc[c];
+    }
+    uint64_t sb = 0;
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const bool in = k0 + u < ksn;
+        if (in) *(uint4 *)(pw + ((rt * ksn + k0 + u) * 64 + lane) * 16) = v[u];
+        sb |= (uint64_t)(in ? b[u] : 127u) << (8 * u);
+    }
+    uint8_t *po = ps + (gi * 64 + lane) * 8;
+    if (((uintptr_t)ps & 7) == 0) {
+        *(uint64_t *)po = sb;
+    } else {
+#pragma unroll
+        for (int u = 0; u < 8; u++) po[u] = (uint8_t)(sb >> (8 * u));
+    }
 }
 
 }  // namespace ws
@@ -46,18 +65,9 @@ int ws_prepack_fp4(const uint8_t *w, const uint8_t *s, int64_t rows, int64_t col
     if (!w || !s || !pw || !ps || rows <= 0 || cols <= 0) return WS_ERR_INVALID_ARG;
     if (rows % 16 || cols % 128 || cols > (1 << 24)) return WS_ERR_SHAPE;
     if (((uintptr_t)w | (uintptr_t)pw) & 15) return WS_ERR_INVALID_ARG;
-    const int64_t n = rows * (cols / 32);
-    // the padding bytes of every lane's last 8-step scale group are never
-    // read; fill them anyway so the packed buffer is deterministic
-    const int64_t sb = packed_fp4_scale_bytes(rows, cols);
-    if ((cols / 128) % 8) {
-        hipLaunchKernelGGL(fill_u8_kernel, dim3((unsigned)((sb + 255) / 256)), dim3(256), 0, stream,
-                           ps, sb, (uint8_t)127);
-        int rc = launch_status();
-        if (rc) return rc;
-    }
-    hipLaunchKernelGGL(prepack_fp4_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
-                       w, s, pw, ps, rows, (int)cols);
+    const int64_t groups = (rows / 16) * ((cols / 128 + 7) / 8);
+    hipLaunchKernelGGL(prepack_fp4_kernel, dim3((unsigned)((groups + 3) / 4)), dim3(256), 0, stream,
+                       w, s, pw, ps, groups, (int)cols);
     return launch_status();
 }
 
