@@ -131,7 +131,7 @@ int ws_fp8_gemm(const uint8_t *a, const uint8_t *sa, const uint8_t *b, const uin
  * engine's gemm_q8 of wo_b, engine.rs:4008-4017) followed by launch.rs:1175
  * acc_f32 into the residual, in one launch: c += A.B^T with the add in the
  * GEMM's epilogue (c[i] + sum). Same operands as ws_fp8_gemm. It runs the
- * line and column-strip kernels only, never split over K: its bits are
+ * line, column-strip and whole-K tile kernels, never split over K: its bits are
  * those of ws_fp8_gemm + ws_acc_f32 wherever ws_fp8_gemm runs those too
  * (m <= 64, or K a multiple of 512 with m <= 128 and one round of tiles;
  * not where it splits K over a registered workspace or runs the split-K

@@ -523,3 +523,117 @@ def test_line_gemm_ragged_rows_vs_fp64_dequant(m, n, k, native):
         assert_close(host(outf), want_f, tol, "line gemm f32s %dx%dx%d" % (m, n, k))
     finally:
         L.set_math_mode(prev)
+
+
+@pytest.mark.parametrize("m,n,k", [(129, 400, 128), (200, 528, 256), (777, 4608, 384),
+                                   (2000, 4096, 512), (4090, 4080, 640), (65, 4096, 1152)])
+def test_tile_gemm_edges_vs_fp64_dequant(m, n, k):
+    """The whole-K tile kernel in each of its tilings (64 x 128, 128 x 128,
+    128 x 256, 256 x 256) with ragged rows, columns and step counts (1, 2, 3, 4,
+    5 and 9 steps, so that scale groups of four end anywhere), every weight
+    format and epilogue. f32 sums of at most 36 MFMAs: each rounding is at most
+    2^-24 of a partial sum, so the 2-norm error stays under sqrt(36) 2^-24 =
+    3.6e-7; bf16 and accumulating outputs are the f32 result's bits."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(m + n + k)
+    announce("tile gemm m=%d n=%d k=%d" % (m, n, k))
+    x = torch.randn((m, k), device=DEV, generator=gen)
+    w = torch.randn((n, k), device=DEV, generator=gen) * 0.02
+    aq = torch.empty((m, k), dtype=torch.uint8, device=DEV)
+    as_ = torch.empty((m, k // 32), dtype=torch.uint8, device=DEV)
+    L.emit8(x, aq, as_, m * k)
+    wq = torch.empty((n, k), dtype=torch.uint8, device=DEV)
+    ws = torch.empty(((n + 31) // 32, k // 32), dtype=torch.uint8, device=DEV)
+    L.weight_quant_fp8(w, wq, ws, n, k)
+    w4 = torch.empty((n, k // 2), dtype=torch.uint8, device=DEV)
+    s4 = torch.empty((n, k // 32), dtype=torch.uint8, device=DEV)
+    L.weight_quant_fp4(w, w4, s4, n, k)
+    table = torch.from_numpy(O.e4m3_decode_table().astype(np.float64)).to(DEV)
+    pw = lambda s: torch.pow(2.0, s.to(torch.float64) - 127)
+    codes, da = table[aq.long()], None
+    da = codes * pw(as_).repeat_interleave(32, 1)
+    dw = table[wq.long()] * pw(ws).repeat_interleave(32, 0)[:n].repeat_interleave(32, 1)
+
+    def run(call, dtype=torch.float32, start=None):
+        buf = torch.full((m * n + 64,), -7.0, dtype=torch.float32, device=DEV).to(dtype)
+        if start is not None:
+            buf[:m * n] = start.view(-1)
+        call(buf)
+        torch.cuda.synchronize()
+        assert (buf[m * n:] == -7).all(), "written past the output"
+        return buf[:m * n].view(m, n)
+
+    def close(got, want, what):
+        err = float((got.double() - want).norm() / want.norm())
+        print("[tile %s %dx%dx%d] rel 2-norm err %.3g" % (what, m, n, k, err))
+        assert err <= 3.6e-7, (what, err)
+
+    out = run(lambda o: L.fp8_gemm(aq, as_, wq, ws, o, m, n, k))
+    close(out, da @ dw.T, "fp8")
+    ob = run(lambda o: L.fp8_gemm_bf16(aq, as_, wq, ws, o, m, n, k), torch.bfloat16)
+    if m > 128:  # at most 128 rows ws_fp8_gemm may take the line kernel for both
+        assert torch.equal(ob, out.bfloat16())
+        c0 = torch.randn((m, n), device=DEV, generator=gen)
+        acc = run(lambda o: L.fp8_gemm_acc(aq, as_, wq, ws, o, m, n, k), start=c0)
+        assert torch.equal(acc, c0 + out)
+    af = torch.rand((m, k // 128), device=DEV, generator=gen) * 0.01 + 1e-3
+    wf = torch.rand(((n + 127) // 128, k // 128), device=DEV, generator=gen) * 1e-4 + 1e-5
+    fout = run(lambda o: L.fp8_gemm_f32s(aq, af, wq, wf, o, m, n, k))
+    want = ((codes * af.double().repeat_interleave(128, 1))
+            @ (table[wq.long()] * wf.double().repeat_interleave(128, 0)[:n].repeat_interleave(128, 1)).T)
+    close(fout, want, "f32s")
+    lut = torch.tensor([O.fp4_value(i) for i in range(16)], dtype=torch.float64, device=DEV)
+    d4 = torch.stack((lut[(w4 & 15).long()], lut[(w4 >> 4).long()]), -1).view(n, k)
+    got = run(lambda o: L.fp4_gemm(aq, as_, w4, s4, o, m, n, k))
+    close(got, da @ (d4 * pw(s4).repeat_interleave(32, 1)).T, "fp4")
+
+
+@pytest.mark.parametrize("m", [65, 130, 520])
+def test_tile_gemm_packed_scale_table(m):
+    """ws_fp8_gemm_tl above 64 rows: per-row weight scale words, each row with
+    scales of its own, against f64."""
+    kind = L.TL_QB
+    n, k = L.tl_gemm_shape(kind)
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(m)
+    announce("tile gemm tl m=%d" % m)
+    x = torch.randn((m, k), device=DEV, generator=gen)
+    aq = torch.empty((m, k), dtype=torch.uint8, device=DEV)
+    as_ = torch.empty((m, k // 32), dtype=torch.uint8, device=DEV)
+    L.emit8(x, aq, as_, m * k)
+    wq = torch.randint(0, 120, (n, k), dtype=torch.uint8, device=DEV, generator=gen)
+    ws = torch.randint(110, 124, (n, k // 32), dtype=torch.uint8, device=DEV, generator=gen)
+    out = torch.empty((m, n), device=DEV)
+    L.fp8_gemm_tl(kind, aq, as_, wq, ws, out, m)
+    table = torch.from_numpy(O.e4m3_decode_table().astype(np.float64)).to(DEV)
+    pw = lambda s: torch.pow(2.0, s.to(torch.float64) - 127)
+    want = (table[aq.long()] * pw(as_).repeat_interleave(32, 1)) @ \
+        (table[wq.long()] * pw(ws).repeat_interleave(32, 1)).T
+    err = float((out.double() - want).norm() / want.norm())
+    assert err <= 40 ** 0.5 * 2.0 ** -24, err
+
+
+def test_tile_gemm_special_scales_match_strips():
+    """Scale bytes 0 (2^-127) and 255 (NaN) and NaN codes: the tile kernel's
+    rows against the strips that the same rows take 64 at a time."""
+    m, n, k = 256, 512, 640
+    rng = np.random.default_rng(77)
+    aq = rng.integers(0, 256, (m, k)).astype(np.uint8)
+    aq[aq % 128 == 127] = 0x30
+    aq[5, 77] = 0x7F
+    as_ = rng.integers(100, 130, (m, k // 32)).astype(np.uint8)
+    as_[9, 3], as_[10, 4], as_[70] = 0, 255, 0
+    wq = rng.integers(0, 126, (n, k)).astype(np.uint8)
+    ws = rng.integers(100, 130, (n // 32, k // 32)).astype(np.uint8)
+    ws[2, 1], ws[3, 2] = 0, 255
+    announce("tile gemm special scales")
+    a, sa, w, sw = dev(aq), dev(as_), dev(wq), dev(ws)
+    got = torch.empty((m, n), device=DEV)
+    L.fp8_gemm(a, sa, w, sw, got, m, n, k)
+    want = torch.empty((m, n), device=DEV)
+    for r in range(0, m, 64):
+        L.fp8_gemm(a[r:r + 64], sa[r:r + 64], w, sw, want[r:r + 64], 64, n, k)
+    g, wt = host(got), host(want)
+    assert np.isnan(wt).any() and np.array_equal(np.isnan(g), np.isnan(wt))
+    ok = ~np.isnan(wt)
+    assert_close(g[ok], wt[ok], 1e-5, "special scales")

@@ -1133,10 +1133,21 @@ static int gemm_dispatch(const uint8_t *a, const void *sa, const uint8_t *b, con
         return WS_ERR_INVALID_ARG;
     int M = (int)m, N = (int)n, K = (int)k;
     const SkWorkspace wsp = sk_ws(stream);
+    const bool exact = math_mode() == WS_MATH_EXACT;
+    auto tiled = [&]() {
+        return tile_gemm(BFP4, SMODE, !BFP4 && sb_div != 32, OMODE, a, sa, b, sb, out, aux, m, n, k,
+                         stream);
+    };
     if (sb_div != 32) {
         // weight scales per row (the reference's packed scale table): the
-        // column-strip kernel only
-        int rc;
+        // column-strip kernel, and whole-K tiles for more than 64 rows when
+        // the strips are more than one round of workgroups (K = 5120, strips /
+        // tiles, us: M = 96 N = 4608 49.5 / 37, M = 300 N = 2304 57 / 35, M =
+        // 777 N = 4608 210 / 50; one round, M = 100 N = 512, 31 / 38)
+        int rc = -1;
+        // (K > 8192 stays refused there: the strips cannot stage it)
+        if (M > 64 && exact && K <= 8192 && (long)(N / 16) * ((M + 127) / 128) > cu_count()) rc = tiled();
+        if (rc >= 0) return rc;
         if (M <= 16) {
             const int S = kAccOut ? 1 : strip_splits(M, N, K, wsp.ptr ? wsp.bytes : 0);
             rc = launch_kp<1, 1, 1, 8, BFP4, SMODE, OMODE, 1>(a, sa, b, sb, out, M, N, K, stream, S,
@@ -1220,7 +1231,24 @@ static int gemm_dispatch(const uint8_t *a, const void *sa, const uint8_t *b, con
             if (lc >= 0) rc = line_gemm(SMODE, OMODE, a, sa, b, sb, out, M, N, K, stream, lc, aux);
         }
         if (rc >= 0) return rc;
-        // 4. M > 64: the pipelined split-K kernel (128-row tiles)
+        // 4. M > 64, exact math: whole-K tiles (gemm_tile.hip) when they keep
+        // the chip busy: 192 tiles of 128 x 128, 96 at K <= 4096, any number at
+        // K <= 2048 (where the split's partials and their reduction cost more
+        // than the idle CUs). Split-K pipeline against tiles, us: M = 4096,
+        // N = 4096, K = 8192 372 / 197; M = 777, N = 4608, K = 5120 75 / 50 (252
+        // tiles); M = 2000, N = 1280, K = 5120 41 / 47 (160); M = 1024, N =
+        // 2048, K = 4096 33 / 30 (128); M = 200, N = 4096, K = 4096 26 / 29 (64);
+        // M = 200, N = 8192, K = 1280 24 / 13 (128). The accumulating
+        // epilogues have no split to compare with (K > 8192 stays refused there).
+        if (M > 64 && exact) {
+            const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+            if (kAccOut ? K <= 8192 : t128 * 4 >= 3l * cu_count() || K <= 2048 ||
+                (K <= 4096 && t128 * 8 >= 3l * cu_count()))
+                rc = tiled();
+        }
+        if (rc >= 0) return rc;
+        // 5. the other shapes with M > 64: the pipelined split-K kernel
+        // (128-row tiles)
         if (M > 64 && !kAccOut) {
             const int bn = pipe_bn(M, N);
             rc = bn == 256   ? launch_pipe<256, BFP4, SMODE, OMODE>(a, sa, b, sb, out, M, N, K, stream, wsp)
@@ -1228,7 +1256,7 @@ static int gemm_dispatch(const uint8_t *a, const void *sa, const uint8_t *b, con
                              : launch_pipe<64, BFP4, SMODE, OMODE>(a, sa, b, sb, out, M, N, K, stream, wsp);
         }
         if (rc >= 0) return rc;
-        // 5. 16-column strips (no split-K workspace, or shapes the others
+        // 6. 16-column strips (no split-K workspace, or shapes the others
         // do not stage)
         if (M <= 16) {
             const int S = kAccOut ? 1 : strip_splits(M, N, K, wsp.ptr ? wsp.bytes : 0);

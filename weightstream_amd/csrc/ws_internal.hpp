@@ -46,6 +46,11 @@ int gate_w13_launch(const float *h, const float *gw, float *logits, const uint8_
 int line_gemm(int smode, int omode, const uint8_t *a, const void *sa, const uint8_t *b,
               const void *sb, void *out, int m, int n, int k, hipStream_t stream, int cfg,
               const float *aux = nullptr);
+// gemm_tile.hip: the exact-math FP8 / FP4 GEMM for many rows (whole-K tiles); sbrow: FP8 weight scales per row instead of per 32 rows.
+// -1 when the shape, alignment or output mode does not fit.
+int tile_gemm(bool bfp4, int smode, bool sbrow, int omode, const uint8_t *a, const void *sa,
+              const uint8_t *b, const void *sb, void *out, const float *aux, int64_t m, int64_t n,
+              int64_t k, hipStream_t stream);
 // C = C + (aux + A.B^T) with UE8M0 32 x 32 weight scales (gemm.hip)
 int fp8_gemm_acc2(const uint8_t *a, const uint8_t *sa, const uint8_t *b, const uint8_t *sb,
                   float *c, const float *aux, int64_t m, int64_t n, int64_t k, hipStream_t stream);
