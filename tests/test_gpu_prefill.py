@@ -159,6 +159,16 @@ def test_moe_prefill_matches_oracle(m, E, dim, inter, k, check):
         _check_by_stages(gy[r], x[r], gi[r], gw[r], H, staged, r, k, dim, inter)
 
 
+@pytest.mark.parametrize("m,E,dim,inter,k", [(120, 16, 768, 384, 4), (200, 32, 2304, 1152, 6),
+                                             (300, 24, 1280, 640, 4), (130, 8, 256, 128, 2),
+                                             (100, 64, 5120, 2432, 6)])
+def test_moe_prefill_stationary_step_counts(m, E, dim, inter, k):
+    """The expert-stationary pair with units of every remainder of four 128-K
+    steps (6 and 3, 18 and 9, 10 and 5, 2 and 1, 40 and 19): a unit's repeated
+    steps past K multiply nothing. Skewed enough that the dispatch takes it."""
+    test_moe_prefill_matches_oracle(m, E, dim, inter, k, 6)
+
+
 @pytest.mark.parametrize("m,check", [(132, 12), (300, 12), (4500, 8)])
 def test_prefill_all_routes_on_k_experts(m, check):
     """Every token picks the same k experts (their bias lifts them above the

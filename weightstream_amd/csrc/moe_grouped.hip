@@ -1058,7 +1058,12 @@ __device__ __forceinline__ void es_lds_get2(uint32_t a, float &v0, float &v1) {
 // MODE 0: gate/up + SwiGLU + routing weight + FP8 1x32 re-quantisation of h,
 // written as the exact bf16 of the quantised values (the down step's A).
 // MODE 1: down, f32 out for the slots that hold routes.
-template <int MODE>
+// PAD: K is not whole rounds of the ring (8 steps); a unit is then a multiple
+// of four steps, the ones past K repeating its last loads and multiplying
+// nothing (K = 2304: 18 steps and two). Without it the unit's end is one place
+// in the code and no step tests for it: 132 tokens at Zipf(1.1) 190 against
+// 196 us.
+template <int MODE, bool PAD>
 __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
     using namespace es;
     constexpr int kAhead = 6;  // steps issued ahead of the one multiplied
@@ -1071,7 +1076,8 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
     const int t = threadIdx.x, lane = t & 63;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int r = lane & 15, g = lane >> 4;
-    const int NS = a.K / 128;                            // steps per unit
+    const int NS = a.K / 128;
+    const int NSP = PAD ? (NS + 3) & ~3 : NS;  // steps per unit
     const int NCG = MODE == 0 ? a.N / 128 : a.N / 256;  // column blocks per group
     const int nt = min(*a.num_tiles, min(kMaxGroups, a.slots / kTile));
 
@@ -1148,7 +1154,7 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
     auto unit_k = [&](int ri) { return ri * G + ((ri & 1) ? G - 1 - pb : pb); };
     const int n_units = U / G + (unit_k(U / G) < U ? 1 : 0);
     if (n_units == 0) return;  // whole workgroup
-    const int total = n_units * NS;
+    const int total = n_units * NSP;
     const size_t wmat = (size_t)a.N * (a.K / 2);
     const size_t smat = (size_t)packed_fp4_scale_bytes(a.N, a.K);
     const uint32_t ring = lds_addr(g_lds);
@@ -1224,19 +1230,20 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
     // of the stream (real == false) the last step's loads are repeated and
     // not used, so that every step has the same loads in flight after it.
     auto issue = [&](EsStep &x, int slot, bool real) {
+        const int sl = PAD ? min(s_i, NS - 1) : s_i;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const int m = MODE == 0 ? h : 0;
             x.q[h] = __builtin_bit_cast(
-                u32x4v, __builtin_amdgcn_raw_buffer_load_b128(wr[m], bo[h] + (uint32_t)s_i * 1024u, 0, 0));
+                u32x4v, __builtin_amdgcn_raw_buffer_load_b128(wr[m], bo[h] + (uint32_t)sl * 1024u, 0, 0));
         }
         const uint32_t lb = ring + slot * kSlotB + 4 * w * kRowB;
 #pragma unroll
         for (int j = 0; j < kTG; j++)
             if ((cmask >> j) & 1)  // uniform: tiles the group has, rows with routes
-                es_dma(abuf, ao[j] + (uint32_t)s_i * kRowB, lb + j * kTile * kRowB, 16);
+                es_dma(abuf, ao[j] + (uint32_t)sl * kRowB, lb + j * kTile * kRowB, 16);
         nT[slot] = __builtin_popcount(cmask);
-        if (real && ++s_i == NS) {
+        if (real && ++s_i == NSP) {
             s_i = 0;
             ri_i++;
         }
@@ -1296,6 +1303,7 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
 #pragma unroll
                 for (int h = 0; h < 2; h++) acc[j][h][0] = acc[j][h][1] = v4f{0.f, 0.f, 0.f, 0.f};
         }
+        if (PAD && s_c >= NS) return;  // uniform: a step past K
         v8bf bq[2][4];
 #pragma unroll
         for (int h = 0; h < 2; h++)
@@ -1421,9 +1429,9 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
         }
     };
 
-    // ---- the stream, unrolled by the ring (static register slots); NS is a
-    // multiple of kRing, so units end on the last step of an iteration. Every
-    // step issues one step (past the end a repeat), and steps 3 and 7 of an
+    // ---- the stream, unrolled by the ring (static register slots); a unit is a
+    // multiple of kRing steps (PAD: of four), so it ends at the last step (or
+    // the fourth) of an iteration. Every step issues one step (past the end a repeat), and steps 3 and 7 of an
     // iteration load a block of scale words, so when steps q and q + 1 are
     // waited for, the loads of steps q + 2 .. q + kAhead - 1 and the scale
     // loads at the ends of steps q - 5 .. q - 1 are newer.
@@ -1433,10 +1441,14 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
     open_compute();
 #pragma unroll
     for (int u = 0; u < kAhead; u++) {
-        if (s_i == 0) open_issue();
-        issue(st[u], u, true);
+        // a stream of one four-step unit ends here: there is no next unit to open
+        const bool real = !PAD || u < total;
+        if (real && s_i == 0) open_issue();
+        issue(st[u], u, real);
+        // steps 0 .. 3, while the issue side is still in their unit (a unit of
+        // four steps is followed by the next one's steps 4 and 5)
+        if (u == 3) load_scales(0, 4);
     }
-    load_scales(0, 6);  // steps 0 .. 3
     load_scales(1, 2);  // steps 4 .. 7
     auto step = [&](EsStep &x, EsStep &next, int u, int q) {
         if ((u & 1) == 0) {
@@ -1456,21 +1468,27 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
         s_c++;
     };
     static_assert(kRing == 8 && kAhead <= kRing - 2, "eight ring slots, slot q - 2 the newest reused");
+    auto unit_end = [&]() {
+        if (s_c != NSP) return;
+        epilogue();
+        s_c = 0;
+        ri_c++;
+        if (ri_c < n_units) open_compute();
+    };
     for (int q = 0; q < total; q += kRing) {
         step(st[0], st[(0 + kAhead) % kRing], 0, q);
         step(st[1], st[(1 + kAhead) % kRing], 1, q + 1);
         step(st[2], st[(2 + kAhead) % kRing], 2, q + 2);
         step(st[3], st[(3 + kAhead) % kRing], 3, q + 3);
+        if constexpr (PAD) {
+            unit_end();
+            if (q + 4 >= total) break;
+        }
         step(st[4], st[(4 + kAhead) % kRing], 4, q + 4);
         step(st[5], st[(5 + kAhead) % kRing], 5, q + 5);
         step(st[6], st[(6 + kAhead) % kRing], 6, q + 6);
         step(st[7], st[(7 + kAhead) % kRing], 7, q + 7);
-        if (s_c == NS) {
-            epilogue();
-            s_c = 0;
-            ri_c++;
-            if (ri_c < n_units) open_compute();
-        }
+        unit_end();
     }
     // the repeated loads of the last steps end here
     es_vmcnt<0>();
@@ -1487,28 +1505,28 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
 // One launch per half of the prefill that runs the expert-stationary body
 // when the dispatch found that its groups pay (*select, es_pays) and the
 // tile-streaming body otherwise; every workgroup takes the same branch.
-template <int ROWS, int CB>
+template <int ROWS, int CB, bool PAD>
 __global__ __launch_bounds__(kGThreads) void glu_select_kernel(const int32_t *select, EsArgs ea,
                                                               GluArgs ga) {
     extern __shared__ __align__(16) uint8_t g_lds[];
-    if (__builtin_amdgcn_readfirstlane(*select)) es_body<0>(ea, g_lds);
+    if (__builtin_amdgcn_readfirstlane(*select)) es_body<0, PAD>(ea, g_lds);
     else grouped_glu_body<true, ROWS, CB>(ga, g_lds);
 }
 
-template <int CB, bool ABF>
+template <int CB, bool ABF, bool PAD>
 __global__ __launch_bounds__(kGThreads) void down_select_kernel(const int32_t *select, EsArgs ea,
                                                                DownArgs da) {
     extern __shared__ __align__(16) uint8_t g_lds[];
-    if (__builtin_amdgcn_readfirstlane(*select)) es_body<1>(ea, g_lds);
+    if (__builtin_amdgcn_readfirstlane(*select)) es_body<1, PAD>(ea, g_lds);
     else grouped_down_body<true, CB, false, ABF>(da, g_lds);
 }
 
 // The expert-stationary pair serves exact math, dim a multiple of 256 (whole
-// 256-column down blocks), K steps (dim / 128, inter / 128) in whole rounds of
-// the ring and at most kMaxGroups tiles.
+// 256-column down blocks) and at most kMaxGroups tiles. 600 tokens, 384
+// experts, top-6, dim 5120, inter 2304 (the tile-streaming pair read each
+// 16-row half of a tile's weights again above dim 4096): 2200 -> 1383 us.
 static bool es_fits(int64_t dim, int64_t inter, int64_t tiles) {
     return math_mode() == WS_MATH_EXACT && dim % 256 == 0 && inter % 128 == 0 &&
-           (dim / 128) % es::kRing == 0 && (inter / 128) % es::kRing == 0 &&
            tiles <= es::kMaxGroups;
 }
 
@@ -1874,13 +1892,16 @@ int ws_moe_prefill(const float *x, const int32_t *topk_idx, const float *topk_w,
         const bool wide = wide_units(tiles);
         const int grows = dim <= 4096 ? 32 : 16;
         const size_t glds = std::max(es::kLdsAll, g_tile_lds(grows, (int)dim));
+#define WS_GLU_SEL(R, W, P) \
+    hipLaunchKernelGGL((glu_select_kernel<R, W, P>), grid, dim3(kGThreads), glds, stream, sel, ea, ga)
+#define WS_GLU_SEL_P(R, W) { if (dim / 128 % es::kRing) WS_GLU_SEL(R, W, true); else WS_GLU_SEL(R, W, false); }
         if (grows == 32) {
-            if (wide) hipLaunchKernelGGL((glu_select_kernel<32, 2>), grid, dim3(kGThreads), glds, stream, sel, ea, ga);
-            else hipLaunchKernelGGL((glu_select_kernel<32, 1>), grid, dim3(kGThreads), glds, stream, sel, ea, ga);
+            if (wide) WS_GLU_SEL_P(32, 2) else WS_GLU_SEL_P(32, 1)
         } else {
-            if (wide) hipLaunchKernelGGL((glu_select_kernel<16, 2>), grid, dim3(kGThreads), glds, stream, sel, ea, ga);
-            else hipLaunchKernelGGL((glu_select_kernel<16, 1>), grid, dim3(kGThreads), glds, stream, sel, ea, ga);
+            if (wide) WS_GLU_SEL_P(16, 2) else WS_GLU_SEL_P(16, 1)
         }
+#undef WS_GLU_SEL_P
+#undef WS_GLU_SEL
         if ((rc = launch_status())) return rc;
         const EsArgs eb{(const uint8_t *)hbf, order, layout_w, tile_expert, ntiles, off, cnt,
                         w2, s2, nullptr, nullptr, nullptr, down, (int)inter, (int)dim,
@@ -1890,13 +1911,16 @@ int ws_moe_prefill(const float *x, const int32_t *topk_idx, const float *topk_w,
         const bool abf = inter <= kAbfMaxK;
         const size_t dlds = std::max(es::kLdsAll, abf ? g_abf_lds(kTile, (int)inter)
                                                       : g_tile_lds(kTile, (int)inter));
+#define WS_DOWN_SEL(W, A, P) \
+    hipLaunchKernelGGL((down_select_kernel<W, A, P>), grid, dim3(kGThreads), dlds, stream, sel, eb, da)
+#define WS_DOWN_SEL_P(W, A) { if (inter / 128 % es::kRing) WS_DOWN_SEL(W, A, true); else WS_DOWN_SEL(W, A, false); }
         if (abf) {
-            if (wide) hipLaunchKernelGGL((down_select_kernel<2, true>), grid, dim3(kGThreads), dlds, stream, sel, eb, da);
-            else hipLaunchKernelGGL((down_select_kernel<1, true>), grid, dim3(kGThreads), dlds, stream, sel, eb, da);
+            if (wide) WS_DOWN_SEL_P(2, true) else WS_DOWN_SEL_P(1, true)
         } else {
-            if (wide) hipLaunchKernelGGL((down_select_kernel<2, false>), grid, dim3(kGThreads), dlds, stream, sel, eb, da);
-            else hipLaunchKernelGGL((down_select_kernel<1, false>), grid, dim3(kGThreads), dlds, stream, sel, eb, da);
+            if (wide) WS_DOWN_SEL_P(2, false) else WS_DOWN_SEL_P(1, false)
         }
+#undef WS_DOWN_SEL_P
+#undef WS_DOWN_SEL
         if ((rc = launch_status())) return rc;
         return ws_moe_combine_f32(down, route_pos, y, dim, top_k, rows, tiles, stream);
     }
