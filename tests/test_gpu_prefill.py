@@ -169,6 +169,18 @@ def test_moe_prefill_stationary_step_counts(m, E, dim, inter, k):
     test_moe_prefill_matches_oracle(m, E, dim, inter, k, 6)
 
 
+@pytest.mark.parametrize("m,E,dim,inter,k", [(600, 16, 768, 384, 4), (1000, 32, 1280, 640, 4),
+                                             (4600, 64, 512, 256, 8), (700, 8, 2304, 1152, 2),
+                                             (260, 3, 640, 128, 3)])
+def test_moe_prefill_group_tiles(m, E, dim, inter, k):
+    """The 96-slot groups (64 or more routes per expert): experts with no route,
+    fewer than 32, every strip count and several groups; step counts of every
+    remainder of four (6 and 3, 10 and 5, 4 and 2, 18 and 9, 5 and 1); column
+    blocks cut short (inter 384, 640, 1152, 128 of 256; dim 768, 1280, 2304, 640
+    of 512)."""
+    test_moe_prefill_matches_oracle(m, E, dim, inter, k, 6)
+
+
 @pytest.mark.parametrize("m,check", [(132, 12), (300, 12), (4500, 8)])
 def test_prefill_all_routes_on_k_experts(m, check):
     """Every token picks the same k experts (their bias lifts them above the

@@ -22,7 +22,7 @@ LIB = os.path.join(PKG, "libweightstream_hip.so")
 LIB_NATIVE = os.path.join(PKG, "libweightstream_hip_native.so")
 
 SOURCES = ["common.hip", "pack.hip", "gemm.hip", "gemm_line.hip", "gemm_tile.hip", "moe_route.hip", "moe_decode.hip", "moe_grouped.hip",
-           "moe_shared.hip"]
+           "moe_shared.hip", "moe_tile.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

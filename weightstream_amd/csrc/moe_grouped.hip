@@ -62,14 +62,34 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(
     uint16_t *__restrict__ xbf, int32_t *__restrict__ select_out) {
     if (blockIdx.x > 0) {
         // workgroups 1..: the tokens' FP8 1x32 quantisation (the act_quant
-        // rule, a 32-lane half-wave per block; nx % 32 == 0), independent of
-        // the dispatch and run beside it in the same launch; with xbf also
-        // the exact bf16 of each quantised value (byte times block scale)
-        const int64_t i = (int64_t)(blockIdx.x - 1) * kDispThreads + threadIdx.x;
-        const bool live = i < nx;
-        uint32_t sb;
-        const uint32_t qb = quant_fp8_block32(live ? xf[i] : 0.0f, &sb);
-        if (live) {
+        // rule, nx % 32 == 0), independent of the dispatch and run beside it in
+        // the same launch; with xbf also the exact bf16 of each quantised value
+        // (byte times block scale). Four values per lane, a block being 8 lanes,
+        // when xf is 16-byte aligned (one 4-byte store per lane, not one byte), else one
+        // and a half-wave.
+        if (((uintptr_t)xf & 15) == 0) {
+            const int64_t i = ((int64_t)(blockIdx.x - 1) * kDispThreads + threadIdx.x) * 4;
+            const bool live = i < nx;
+            uint32_t sb;
+            const float4 v = live ? *(const float4 *)(xf + i) : float4{0.f, 0.f, 0.f, 0.f};
+            const uint32_t qb = quant_fp8_block32_x4(v, &sb);
+            if (!live) return;
+            *(uint32_t *)(xq + i) = qb;
+            if ((threadIdx.x & 7) == 0) xs[i / 32] = (uint8_t)sb;
+            if (xbf) {
+                const float sc = e8m0_to_f32(sb);
+                *(uint2 *)(xbf + i) =
+                    uint2{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(qb, sc, false)),
+                          __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(qb, sc, true))};
+            }
+            return;
+        }
+        for (int64_t i = (int64_t)(blockIdx.x - 1) * kDispThreads * 4 + threadIdx.x, k = 0; k < 4;
+             k++, i += kDispThreads) {
+            const bool live = i < nx;
+            uint32_t sb;
+            const uint32_t qb = quant_fp8_block32(live ? xf[i] : 0.0f, &sb);
+            if (!live) continue;
             xq[i] = (uint8_t)qb;
             if ((threadIdx.x & 31) == 0) xs[i / 32] = (uint8_t)sb;
             if (xbf)
@@ -99,14 +119,10 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(
     __syncthreads();
     // pass 1: stable rank of every route inside its expert (chunk by chunk,
     // in route order)
-    auto rank_chunk = [&](int e) {
-        const bool valid = e >= 0;
-#pragma unroll
-        for (int ww = 0; ww < kDispThreads / 64; ww++) wcnt[ww][t] = 0;
-        __syncthreads();
-        // the wave's lanes with the same expert: the AND over the id's bits
-        // (n_experts <= 1024: 10 bits, and the sign for -1) of the ballot of
-        // lanes that agree with this lane on that bit
+    // the wave's lanes with the same expert: the AND over the id's bits
+    // (n_experts <= 1024: 10 bits, and the sign for -1) of the ballot of
+    // lanes that agree with this lane on that bit
+    auto match = [&](int e) {
         uint64_t same = ~0ull;
 #pragma unroll
         for (int b = 0; b < 11; b++) {
@@ -114,6 +130,14 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(
             const uint64_t m = __ballot(bit);
             same &= bit ? m : ~m;
         }
+        return same;
+    };
+    auto rank_chunk = [&](int e) {
+        const bool valid = e >= 0;
+#pragma unroll
+        for (int ww = 0; ww < kDispThreads / 64; ww++) wcnt[ww][t] = 0;
+        __syncthreads();
+        const uint64_t same = match(e);
         const int cnt = __popcll(same);
         const int inrank = __popcll(same & ((1ull << lane) - 1));
         if (valid && inrank == 0) wcnt[w][e] = cnt;
@@ -133,13 +157,55 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(
         __syncthreads();
         return rank;
     };
+    // Many routes: wave w ranks the contiguous routes [w * per, (w + 1) * per) on
+    // counters of its own, so a batch of 64 costs one match and one LDS round
+    // trip and no barrier; the waves' counts are added up once at the end
+    // (32768 routes and their 4096 tokens' quantisation: 113 us with chunks of
+    // 1024 and four barriers each, 97 so).
+    constexpr int kWv = kDispThreads / 64, kUn = 4;
+    const bool many = routes > kDispHeld * kDispThreads;
+    const int per = (routes + kWv * 64 * kUn - 1) / (kWv * 64 * kUn) * 64 * kUn;
+    const int wr0 = w * per, wr1 = min(wr0 + per, routes);
+    if (!many) {
 #pragma unroll
-    for (int h = 0; h < kDispHeld; h++)
-        if (h * kDispThreads < routes) rk_h[h] = rank_chunk(e_h[h]);  // uniform
-    for (int c0 = kDispHeld * kDispThreads; c0 < routes; c0 += kDispThreads) {
-        const int r = c0 + t;
-        const int rank = rank_chunk(r < routes ? id_of(idx[r], n_experts) : -1);
-        if (rank >= 0) route_pos[r] = rank;
+        for (int h = 0; h < kDispHeld; h++)
+            if (h * kDispThreads < routes) rk_h[h] = rank_chunk(e_h[h]);  // uniform
+    } else {
+#pragma unroll
+        for (int ww = 0; ww < kWv; ww++) wcnt[ww][t] = 0;
+        __syncthreads();
+        volatile int32_t *mine = wcnt[w];
+        for (int c = wr0; c < wr1; c += 64 * kUn) {
+            int e[kUn];
+#pragma unroll
+            for (int u = 0; u < kUn; u++) {
+                const int r = c + u * 64 + lane;
+                e[u] = r < wr1 ? id_of(idx[r], n_experts) : -1;
+            }
+#pragma unroll
+            for (int u = 0; u < kUn; u++) {
+                const int r = c + u * 64 + lane;
+                const uint64_t same = match(e[u]);
+                const int inrank = __popcll(same & ((1ull << lane) - 1));
+                if (e[u] >= 0) {  // a wave's LDS accesses complete in order
+                    const int before = mine[e[u]];
+                    if (inrank == 0) mine[e[u]] = before + __popcll(same);
+                    route_pos[r] = before + inrank;
+                }
+            }
+        }
+        __syncthreads();
+        if (t < n_experts) {
+            int run = 0;
+#pragma unroll
+            for (int ww = 0; ww < kWv; ww++) {
+                const int v = wcnt[ww][t];
+                wcnt[ww][t] = run;
+                run += v;
+            }
+            base[t] = run;
+        }
+        __syncthreads();
     }
     // exclusive scan of the 32-padded counts over experts
     const int count = t < n_experts ? base[t] : 0;
@@ -206,14 +272,29 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(
         }
         route_pos[r] = slot;
     };
+    if (!many) {
 #pragma unroll
-    for (int h = 0; h < kDispHeld; h++) {
-        const int r = h * kDispThreads + t;
-        if (r < routes) place(r, e_h[h], rk_h[h], w_h[h]);
+        for (int h = 0; h < kDispHeld; h++) {
+            const int r = h * kDispThreads + t;
+            if (r < routes) place(r, e_h[h], rk_h[h], w_h[h]);
+        }
+        return;
     }
-    for (int r = kDispHeld * kDispThreads + t; r < routes; r += kDispThreads) {
-        const int e = id_of(idx[r], n_experts);
-        place(r, e, e >= 0 ? route_pos[r] : 0, wts[r]);
+    for (int c = wr0; c < wr1; c += 64 * kUn) {
+        int e[kUn], rank[kUn];
+        float wr[kUn];
+#pragma unroll
+        for (int u = 0; u < kUn; u++) {  // the lane that ranked the route reads its rank back
+            const int r = min(c + u * 64 + lane, wr1 - 1);
+            e[u] = id_of(idx[r], n_experts);
+            rank[u] = route_pos[r];
+            wr[u] = wts[r];
+        }
+#pragma unroll
+        for (int u = 0; u < kUn; u++) {
+            const int r = c + u * 64 + lane;
+            if (r < wr1) place(r, e[u], e[u] >= 0 ? wcnt[w][e[u]] + rank[u] : 0, wr[u]);
+        }
     }
 }
 
@@ -1530,9 +1611,25 @@ static bool es_fits(int64_t dim, int64_t inter, int64_t tiles) {
            tiles <= es::kMaxGroups;
 }
 
+// The 96-slot groups of moe_tile.hip: exact math, from 64 routes per expert
+// on, and from 8 where the stationary pair's group table is too small
+// (kMaxGroups tiles). 384 experts, us for the whole prefill, stationary (or, past
+// 1024 tiles, tile-streaming) pair / groups: dim 4096, inter 2048, top-8 at
+// 12.5 / 32 / 42 routes per expert 889 / 985, 1406 / 1355, 1600 / 1520; 62 and
+// 85 (streaming) 2556 / 1414, 3816 / 2191; dim 5120, inter 2304, top-6 at 62
+// (streaming) 5814 / 2437; 96 experts, dim 2304, inter 1152 at 125 420 / 380.
+// The sums, and so the bits, are the stationary pair's.
+static bool mt_pays(int64_t rows, int64_t dim, int64_t inter, int64_t slots, int64_t routes,
+                    int64_t n_experts, int64_t tiles) {
+    if (math_mode() != WS_MATH_EXACT) return false;
+    if (rows * dim * 2 >= (1ll << 32) || slots * inter * 2 >= (1ll << 32)) return false;  // 32-bit rows
+    return routes >= 64 * n_experts || (tiles > es::kMaxGroups && routes >= 8 * n_experts);
+}
+
 // ---- combine: y[row] = sum of its routes' outputs in ascending slot order --
-// V columns per thread (V = 4: 16-byte loads, dim % 4 == 0)
-template <int V>
+// V columns per thread (V = 4: 16-byte loads, dim % 4 == 0; the loads of GRP
+// rows are issued before their ordered adds)
+template <int V, int GRP>
 __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ down,
                                                       const int32_t *__restrict__ route_pos,
                                                       float *__restrict__ y, int dim, int top_k,
@@ -1559,13 +1656,24 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
     const int d = (blockIdx.x * 256 + threadIdx.x) * V;
     if (d >= dim) return;
     if constexpr (V == 4) {
+        // a load per row between the adds left the kernel waiting for each:
+        // 4096 rows of top-8, dim 4096 140 -> 116 us (rows past ns repeat the
+        // group's first and are not added)
         float4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int i = 0; i < ns; i++) {
-            const float4 v = *(const float4 *)(down + (size_t)slots[i] * dim + d);
-            acc.x = acc.x + v.x;
-            acc.y = acc.y + v.y;
-            acc.z = acc.z + v.z;
-            acc.w = acc.w + v.w;
+        const int n = ns;
+        for (int i0 = 0; i0 < n; i0 += GRP) {
+            float4 v[GRP];
+#pragma unroll
+            for (int i = 0; i < GRP; i++)
+                v[i] = *(const float4 *)(down + (size_t)slots[i0 + i < n ? i0 + i : i0] * dim + d);
+#pragma unroll
+            for (int i = 0; i < GRP; i++) {
+                if (i0 + i >= n) break;  // uniform
+                acc.x = acc.x + v[i].x;
+                acc.y = acc.y + v[i].y;
+                acc.z = acc.z + v[i].z;
+                acc.w = acc.w + v[i].w;
+            }
         }
         *(float4 *)(y + (size_t)row * dim + d) = acc;
     } else {
@@ -1628,7 +1736,7 @@ static int dispatch_launch(const int32_t *topk_idx, const float *topk_w, int32_t
                            int64_t n_experts, const float *xf, uint8_t *xq, uint8_t *xs,
                            int64_t nx, ws_stream_t stream, uint16_t *xbf = nullptr,
                            int32_t *select = nullptr) {
-    const int64_t qblocks = (nx + kDispThreads - 1) / kDispThreads;
+    const int64_t qblocks = (nx + 4 * kDispThreads - 1) / (4 * kDispThreads);
     hipLaunchKernelGGL(dispatch_kernel<int32_t>, dim3((unsigned)(1 + qblocks)), dim3(kDispThreads),
                        0, stream, topk_idx, topk_w, order, layout_w, route_pos, tile_expert,
                        expert_count, expert_offset, expert_psum, num_tiles, (int)(rows * top_k),
@@ -1813,14 +1921,21 @@ int ws_moe_combine_f32(const float *y, const int32_t *route_pos, float *out, int
     if (!y || !route_pos || !out) return WS_ERR_INVALID_ARG;
     if (rows <= 0 || dim <= 0 || top_k <= 0 || tiles <= 0) return WS_ERR_INVALID_ARG;
     if (top_k > 16 || rows > 65535) return WS_ERR_SHAPE;
-    if (dim % 4 == 0 && al16(y) && al16(out))
-        hipLaunchKernelGGL(combine_kernel<4>,
-                           dim3((unsigned)((dim / 4 + 255) / 256), (unsigned)rows), dim3(256), 0,
-                           stream, y, route_pos, out, (int)dim, (int)top_k, (int)(tiles * kTile));
-    else
-        hipLaunchKernelGGL(combine_kernel<1>, dim3((unsigned)((dim + 255) / 256), (unsigned)rows),
-                           dim3(256), 0, stream, y, route_pos, out, (int)dim, (int)top_k,
-                           (int)(tiles * kTile));
+    const int cap = (int)(tiles * kTile);
+    if (dim % 4 == 0 && al16(y) && al16(out)) {
+        const dim3 grid((unsigned)((dim / 4 + 255) / 256), (unsigned)rows);
+#define WS_COMBINE(GRP)                                                                        \
+    hipLaunchKernelGGL((combine_kernel<4, GRP>), grid, dim3(256), 0, stream, y, route_pos, out, \
+                       (int)dim, (int)top_k, cap)
+        if (top_k <= 2) WS_COMBINE(2);
+        else if (top_k <= 4) WS_COMBINE(4);
+        else if (top_k <= 6) WS_COMBINE(6);
+        else WS_COMBINE(8);
+#undef WS_COMBINE
+    } else {
+        hipLaunchKernelGGL((combine_kernel<1, 1>), dim3((unsigned)((dim + 255) / 256), (unsigned)rows),
+                           dim3(256), 0, stream, y, route_pos, out, (int)dim, (int)top_k, cap);
+    }
     return launch_status();
 }
 
@@ -1875,11 +1990,21 @@ int ws_moe_prefill(const float *x, const int32_t *topk_idx, const float *topk_w,
     uint16_t *hbf = (uint16_t *)take(slots * inter * 2);
     // the dispatch and the tokens' quantisation in one launch
     if (n_experts > kMaxExpertsG || routes > (1 << 26) || tiles > (1 << 24)) return WS_ERR_SHAPE;
-    const bool stationary = es_fits(dim, inter, tiles);
+    const bool tiled = mt_pays(rows, dim, inter, slots, routes, n_experts, tiles);
+    const bool stationary = !tiled && es_fits(dim, inter, tiles);
     int rc = dispatch_launch(topk_idx, topk_w, order, layout_w, route_pos, tile_expert, cnt, off,
                              psum, ntiles, rows, top_k, tiles, n_experts, x, xq, xs, rows * dim,
-                             stream, stationary ? xbf : nullptr, stationary ? sel : nullptr);
+                             stream, stationary || tiled ? xbf : nullptr, stationary ? sel : nullptr);
     if (rc) return rc;
+    if (tiled) {
+        rc = moe_tile_glu(xbf, order, layout_w, off, cnt, w1, s1, w3, s3, hbf, (int)dim, (int)inter,
+                          (int)n_experts, (int)top_k, swiglu_limit, stream);
+        if (!rc)
+            rc = moe_tile_down(hbf, off, cnt, w2, s2, down, (int)dim, (int)inter, (int)n_experts,
+                               stream);
+        if (rc) return rc;
+        return ws_moe_combine_f32(down, route_pos, y, dim, top_k, rows, tiles, stream);
+    }
     if (stationary) {
         // both halves run the body the dispatch chose on the device (*sel)
         const dim3 grid((unsigned)cu_count());

@@ -51,6 +51,15 @@ int line_gemm(int smode, int omode, const uint8_t *a, const void *sa, const uint
 int tile_gemm(bool bfp4, int smode, bool sbrow, int omode, const uint8_t *a, const void *sa,
               const uint8_t *b, const void *sb, void *out, const float *aux, int64_t m, int64_t n,
               int64_t k, hipStream_t stream);
+// moe_tile.hip: the grouped gate/up (bf16 h out) and down steps over 96-slot
+// groups, exact math; offsets and counts are the dispatch's.
+int moe_tile_glu(const uint16_t *xbf, const int32_t *order, const float *layout_w,
+                 const int32_t *exp_off, const int32_t *exp_cnt, const uint8_t *w1,
+                 const uint8_t *s1, const uint8_t *w3, const uint8_t *s3, uint16_t *hbf, int dim,
+                 int inter, int n_experts, int top_k, float limit, hipStream_t stream);
+int moe_tile_down(const uint16_t *hbf, const int32_t *exp_off, const int32_t *exp_cnt,
+                  const uint8_t *w2, const uint8_t *s2, float *out, int dim, int inter,
+                  int n_experts, hipStream_t stream);
 // C = C + (aux + A.B^T) with UE8M0 32 x 32 weight scales (gemm.hip)
 int fp8_gemm_acc2(const uint8_t *a, const uint8_t *sa, const uint8_t *b, const uint8_t *sb,
                   float *c, const float *aux, int64_t m, int64_t n, int64_t k, hipStream_t stream);
