@@ -282,3 +282,26 @@ def test_device_e4m3_and_activation_scale_equal_oracle_on_every_input():
         ref = np.empty(n, np.uint32)
         O.lib.or_probe_bytes(fn, lo, n, ref.ctypes.data)
         assert np.array_equal(got, ref), fn
+
+
+@pytest.mark.parametrize("m,E,dim,bf16", [(700, 150, 320, False), (700, 150, 320, True),
+                                          (1030, 200, 128, False), (2100, 300, 64, True),
+                                          (4100, 300, 192, False)])
+def test_gate_logits_many_tokens_bit_exact(m, E, dim, bf16):
+    """One expert and 1, 2 or 4 tokens per lane (98304 or more chains): ragged
+    expert blocks and token groups, an odd number of 64-element chunks, f32 and
+    bf16 weights; the sequential f32 dots of the oracle bit for bit."""
+    gen = torch.Generator(device=DEV).manual_seed(m + E)
+    x = torch.randn((m, dim), device=DEV, generator=gen)
+    w = torch.randn((E, dim), device=DEV, generator=gen) * 0.02
+    w = w.bfloat16() if bf16 else w
+    out = torch.full((m * E + 64,), -7.0, device=DEV)
+    announce("gate logits m=%d E=%d dim=%d bf16=%d" % (m, E, dim, bf16))
+    L.moe_gate_logits(x, w, out, m, dim, E)
+    got = host(out)
+    assert (got[m * E:] == -7).all()
+    got = got[:m * E].reshape(m, E)
+    hw, hx = host(w.float()), host(x)
+    for r in sorted({0, 1, 2, 3, 7, m // 2, m - 2, m - 1}):
+        want = O.gemv_f32(hw, hx[r])
+        assert np.array_equal(got[r].view(np.uint32), want.view(np.uint32)), r

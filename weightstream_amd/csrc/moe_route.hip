@@ -242,6 +242,121 @@ static void gate_pipe_launch(const float *x, const void *gw, int bf16, float *lo
                            (int)dim, (int)n_experts);
 }
 
+// ---- gate logits, many tokens (dim % 64 == 0) ----------------------------------
+// A lane owns one expert and T tokens' chains of it (T independent sequential
+// dots of num::gemv, multiply then add: the same bits). The token values are
+// uniform over the wave: a lane holds one element of the chunk per token and
+// v_readlane makes it a scalar operand (through scalar loads instead the chains
+// waited for each: 1024 tokens 205 against 141 us), so only the lane's weight row
+// goes through LDS: one 16-byte read per 4 T products, where a lane with one
+// chain read 32 bytes per 4 and the LDS was the bound. W waves of a workgroup (T
+// tokens each) share the 64 weight rows of a 64-element chunk, staged through
+// registers one chunk ahead of the chains (bf16 weights widened on the way). What
+// bounds it is the vector ALU: three instructions per product, whose waves need
+// company on their SIMD (a lone wave issues one per ~5 cycles, two waves two).
+template <int T, int W, int CH, bool BF16>
+__global__ __launch_bounds__(64 * W) void gate_logits_many_kernel(const float *x, const void *gw,
+                                                                  float *__restrict__ logits,
+                                                                  int m_rows, int dim, int n_experts) {
+    constexpr int kGmChunk = CH, kGmPitch = CH + 4;  // floats; pitch: rows on distinct banks
+    extern __shared__ __align__(16) uint8_t g_lds[];
+    float (*const wl)[64 * kGmPitch] = (float (*)[64 * kGmPitch])g_lds;  // [2]
+    const int t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int e0 = blockIdx.x * 64, m0 = (blockIdx.y * W + w) * T;
+    // staging: thread t copies float4s t, t + 64 W, .. of the 64 rows of a chunk
+    constexpr int kQ = CH / 4, kP = kQ / W;  // float4s per row, per thread
+    static_assert(kQ % W == 0, "whole float4s per thread");
+    v4f st[kP];
+    auto load = [&](int c) {
+#pragma unroll
+        for (int p = 0; p < kP; p++) {
+            const int i = t + p * 64 * W, row = min(e0 + i / kQ, n_experts - 1), q = i % kQ;
+            const size_t o = (size_t)row * dim + c * kGmChunk + 4 * q;
+            if (BF16) {
+                const uint2 v = *(const uint2 *)((const uint16_t *)gw + o);
+                st[p] = v4f{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xFFFF0000u),
+                            __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xFFFF0000u)};
+            } else {
+                st[p] = *(const v4f *)((const float *)gw + o);
+            }
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int p = 0; p < kP; p++) {
+            const int i = t + p * 64 * W;
+            *(v4f *)&wl[buf][i / kQ * kGmPitch + 4 * (i % kQ)] = st[p];
+        }
+    };
+    // a token's chunk, one element per lane and 64
+    float xv[T][CH / 64], xn[T][CH / 64];
+    auto load_x = [&](int c) {
+#pragma unroll
+        for (int j = 0; j < T; j++)
+#pragma unroll
+            for (int k = 0; k < CH / 64; k++)
+                xn[j][k] = x[(size_t)min(m0 + j, m_rows - 1) * dim + c * CH + 64 * k + lane];
+    };
+    float s[T];
+#pragma unroll
+    for (int j = 0; j < T; j++) s[j] = 0.0f;
+    const int nc = dim / kGmChunk;
+    load(0);
+    load_x(0);
+    store(0);
+    __syncthreads();
+    for (int c = 0; c < nc; c++) {
+#pragma unroll
+        for (int j = 0; j < T; j++)
+#pragma unroll
+            for (int k = 0; k < CH / 64; k++) xv[j][k] = xn[j][k];
+        load(min(c + 1, nc - 1));
+        load_x(min(c + 1, nc - 1));
+        // the loads stay here, a chunk of chains ahead of their use
+        mem_order();
+        __builtin_amdgcn_sched_barrier(0);
+        const float *row = &wl[c & 1][lane * kGmPitch];
+#pragma unroll
+        for (int d = 0; d < kGmChunk; d += 4) {
+            const v4f v = *(const v4f *)(row + d);
+            // the products of four elements, then their ordered adds: the chains
+            // of the T tokens alternate
+            float pr[T][4];
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < T; j++)
+                    pr[j][i] = __int_as_float(__builtin_amdgcn_readlane(
+                                   __float_as_int(xv[j][d / 64]), d % 64 + i)) * v[i];
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < T; j++) s[j] = s[j] + pr[j][i];
+        }
+        // the other buffer was read before the last barrier
+        store((c + 1) & 1);
+        __syncthreads();
+    }
+    if (e0 + lane < n_experts)
+#pragma unroll
+        for (int j = 0; j < T; j++)
+            if (m0 + j < m_rows) logits[(size_t)(m0 + j) * n_experts + e0 + lane] = s[j];
+}
+
+template <int T, int W, int CH>
+static void gate_many_launch(const float *x, const void *gw, int bf16, float *logits, int64_t m,
+                             int64_t dim, int64_t n_experts, hipStream_t stream) {
+    const dim3 g((unsigned)((n_experts + 63) / 64), (unsigned)((m + T * W - 1) / (T * W)));
+    constexpr size_t lds = 2 * 64 * (CH + 4) * 4;
+    if (bf16)
+        hipLaunchKernelGGL((gate_logits_many_kernel<T, W, CH, true>), g, dim3(64 * W), lds, stream, x,
+                           gw, logits, (int)m, (int)dim, (int)n_experts);
+    else
+        hipLaunchKernelGGL((gate_logits_many_kernel<T, W, CH, false>), g, dim3(64 * W), lds, stream, x,
+                           gw, logits, (int)m, (int)dim, (int)n_experts);
+}
+
 template <int TE, int TM, bool BF16>
 __global__ __launch_bounds__(128) void gate_logits_pc_kernel(const float *x, const void *gw,
                                                              float *__restrict__ logits,
@@ -409,6 +524,18 @@ static int gate_logits_launch(const float *x, const void *gw, int bf16, float *l
     if (!x || !gw || !logits) return WS_ERR_INVALID_ARG;
     if (m <= 0 || dim <= 0 || n_experts <= 0) return WS_ERR_INVALID_ARG;
     if (dim % 8 || m > 65535 || n_experts > (1 << 20)) return WS_ERR_SHAPE;
+    // many chains: one expert and T tokens per lane; T grows with the waves that
+    // leaves per SIMD (m tokens x blocks of 64 experts). 384 experts, dim 4096, f32
+    // weights, against the 8 x 8 blocks below, us: 128 tokens 52 / 67, 256 79 /
+    // 67, 1024 300 / 141, 2048 595 / 217, 4096 1182 / 394; bf16 1024 256 / 153.
+    if (dim % 64 == 0 && m * n_experts >= 96 * 1024 && ((uintptr_t)gw & 15) == 0) {
+        const int64_t waves = m * ((n_experts + 63) / 64);
+        if (waves <= 3072) gate_many_launch<1, 4, 64>(x, gw, bf16, logits, m, dim, n_experts, stream);
+        else if (waves <= 8192) gate_many_launch<2, 4, 64>(x, gw, bf16, logits, m, dim, n_experts, stream);
+        else if (waves <= 16384) gate_many_launch<2, 8, 64>(x, gw, bf16, logits, m, dim, n_experts, stream);
+        else gate_many_launch<4, 8, 64>(x, gw, bf16, logits, m, dim, n_experts, stream);
+        return launch_status();
+    }
     if (dim % kGC == 0 && m <= (1 << 20)) {
         // one token: 4 experts per wave (the weight stream spread over many
         // CUs); a few tokens: 16 x 4 blocks; more: 8 x 8
