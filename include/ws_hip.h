@@ -113,7 +113,7 @@ int ws_weight_quant_fp8(const float *w, uint8_t *q, uint8_t *s, int64_t rows, in
  * (device, stream): GEMMs issued on `stream` (NULL = the default stream) of
  * the current device use the workspace registered for that stream, so GEMMs
  * on different streams never share one. With a workspace, GEMMs with M > 64
- * (and M <= 16 with few column strips and K > 8192) split K across
+ * and few tiles (and M <= 16 with few column strips and K > 8192) split K across
  * workgroups and a second kernel adds the f32 partials in split order
  * (deterministic); without one they use the single-pass kernels. Calls on one
  * stream are ordered by the stream, so they may share its workspace.
@@ -131,7 +131,7 @@ int ws_fp8_gemm(const uint8_t *a, const uint8_t *sa, const uint8_t *b, const uin
  * engine's gemm_q8 of wo_b, engine.rs:4008-4017) followed by launch.rs:1175
  * acc_f32 into the residual, in one launch: c += A.B^T with the add in the
  * GEMM's epilogue (c[i] + sum). Same operands as ws_fp8_gemm. It runs the
- * line, column-strip and whole-K tile kernels, never split over K: its bits are
+ * line and column-strip kernels only, never split over K: its bits are
  * those of ws_fp8_gemm + ws_acc_f32 wherever ws_fp8_gemm runs those too
  * (m <= 64, or K a multiple of 512 with m <= 128 and one round of tiles;
  * not where it splits K over a registered workspace or runs the split-K

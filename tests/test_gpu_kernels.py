@@ -533,7 +533,9 @@ def test_tile_gemm_edges_vs_fp64_dequant(m, n, k):
     5 and 9 steps, so that scale groups of four end anywhere), every weight
     format and epilogue. f32 sums of at most 36 MFMAs: each rounding is at most
     2^-24 of a partial sum, so the 2-norm error stays under sqrt(36) 2^-24 =
-    3.6e-7; bf16 and accumulating outputs are the f32 result's bits."""
+    3.6e-7; The tiles serve the bf16 output; the f32 and accumulating ones take other
+    kernels whose sums differ in order. Each is within 40 roundings of at most
+    2^-23 of the sum of magnitudes; bf16 adds 2^-8 and the accumulation 2^-23."""
     gen = torch.Generator(device=DEV)
     gen.manual_seed(m + n + k)
     announce("tile gemm m=%d n=%d k=%d" % (m, n, k))
@@ -572,10 +574,12 @@ def test_tile_gemm_edges_vs_fp64_dequant(m, n, k):
     close(out, da @ dw.T, "fp8")
     ob = run(lambda o: L.fp8_gemm_bf16(aq, as_, wq, ws, o, m, n, k), torch.bfloat16)
     if m > 128:  # at most 128 rows ws_fp8_gemm may take the line kernel for both
-        assert torch.equal(ob, out.bfloat16())
+        slack = 2 * 40 * 2.0 ** -23 * (da.abs() @ dw.abs().T)
+        assert ((ob.double() - out.double()).abs() <= 2.0 ** -8 * out.double().abs() + 1.01 * slack).all()
         c0 = torch.randn((m, n), device=DEV, generator=gen)
         acc = run(lambda o: L.fp8_gemm_acc(aq, as_, wq, ws, o, m, n, k), start=c0)
-        assert torch.equal(acc, c0 + out)
+        assert ((acc.double() - c0.double() - out.double()).abs()
+                <= 1.01 * slack + 2.0 ** -23 * (c0 + out).double().abs()).all()
     af = torch.rand((m, k // 128), device=DEV, generator=gen) * 0.01 + 1e-3
     wf = torch.rand(((n + 127) // 128, k // 128), device=DEV, generator=gen) * 1e-4 + 1e-5
     fout = run(lambda o: L.fp8_gemm_f32s(aq, af, wq, wf, o, m, n, k))
@@ -628,12 +632,13 @@ def test_tile_gemm_special_scales_match_strips():
     ws[2, 1], ws[3, 2] = 0, 255
     announce("tile gemm special scales")
     a, sa, w, sw = dev(aq), dev(as_), dev(wq), dev(ws)
-    got = torch.empty((m, n), device=DEV)
-    L.fp8_gemm(a, sa, w, sw, got, m, n, k)
+    got = torch.empty((m, n), device=DEV, dtype=torch.bfloat16)  # what the tiles serve
+    L.fp8_gemm_bf16(a, sa, w, sw, got, m, n, k)
     want = torch.empty((m, n), device=DEV)
     for r in range(0, m, 64):
         L.fp8_gemm(a[r:r + 64], sa[r:r + 64], w, sw, want[r:r + 64], 64, n, k)
-    g, wt = host(got), host(want)
+    g, wt = host(got.float()), host(want)
     assert np.isnan(wt).any() and np.array_equal(np.isnan(g), np.isnan(wt))
     ok = ~np.isnan(wt)
-    assert_close(g[ok], wt[ok], 1e-5, "special scales")
+    # bf16 rounds to within 2^-8 of a value, the f32 sums differ by 1e-5
+    assert_close(g[ok], wt[ok], 2.0 ** -8 + 1e-5, "special scales")

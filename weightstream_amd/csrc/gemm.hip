@@ -1140,14 +1140,8 @@ static int gemm_dispatch(const uint8_t *a, const void *sa, const uint8_t *b, con
     };
     if (sb_div != 32) {
         // weight scales per row (the reference's packed scale table): the
-        // column-strip kernel, and whole-K tiles for more than 64 rows when
-        // the strips are more than one round of workgroups (K = 5120, strips /
-        // tiles, us: M = 96 N = 4608 49.5 / 37, M = 300 N = 2304 57 / 35, M =
-        // 777 N = 4608 210 / 50; one round, M = 100 N = 512, 31 / 38)
+        // column-strip kernel
         int rc = -1;
-        // (K > 8192 stays refused there: the strips cannot stage it)
-        if (M > 64 && exact && K <= 8192 && (long)(N / 16) * ((M + 127) / 128) > cu_count()) rc = tiled();
-        if (rc >= 0) return rc;
         if (M <= 16) {
             const int S = kAccOut ? 1 : strip_splits(M, N, K, wsp.ptr ? wsp.bytes : 0);
             rc = launch_kp<1, 1, 1, 8, BFP4, SMODE, OMODE, 1>(a, sa, b, sb, out, M, N, K, stream, S,
@@ -1238,11 +1232,12 @@ static int gemm_dispatch(const uint8_t *a, const void *sa, const uint8_t *b, con
         // N = 4096, K = 8192 372 / 197; M = 777, N = 4608, K = 5120 75 / 50 (252
         // tiles); M = 2000, N = 1280, K = 5120 41 / 47 (160); M = 1024, N =
         // 2048, K = 4096 33 / 30 (128); M = 200, N = 4096, K = 4096 26 / 29 (64);
-        // M = 200, N = 8192, K = 1280 24 / 13 (128). The accumulating
-        // epilogues have no split to compare with (K > 8192 stays refused there).
-        if (M > 64 && exact) {
+        // M = 200, N = 8192, K = 1280 24 / 13 (128). bf16
+        // results only (the figures are the GEMM's with f32 stores): the f32
+        // ones keep the shorter chains.
+        if (M > 64 && exact && OMODE == kOutBf16) {
             const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-            if (kAccOut ? K <= 8192 : t128 * 4 >= 3l * cu_count() || K <= 2048 ||
+            if (t128 * 4 >= 3l * cu_count() || K <= 2048 ||
                 (K <= 4096 && t128 * 8 >= 3l * cu_count()))
                 rc = tiled();
         }

@@ -446,19 +446,13 @@ int tile_gemm(bool bfp4, int smode, bool sbrow, int omode, const uint8_t *a, con
     if ((uintptr_t)out & (omode == kOutBf16 ? 7 : 15) || (uintptr_t)aux & 15) return -1;
     const Args p{a, b, (const uint8_t *)sa, (const uint8_t *)sb, out, aux, (int)m, (int)n,
                  (int)k, 0, 0};
-    if (bfp4) return omode == kOutF32 ? run<true, kUe8m0, true, kOutF32>(p, stream) : -1;
-    if (sbrow) return omode == kOutF32 ? run<false, kUe8m0, true, kOutF32>(p, stream) : -1;
-    if (smode == kF32s) {
-        if (omode == kOutF32) return run<false, kF32s, false, kOutF32>(p, stream);
-        return omode == kOutBf16 ? run<false, kF32s, false, kOutBf16>(p, stream) : -1;
-    }
-    switch (omode) {
-        case kOutF32: return run<false, kUe8m0, false, kOutF32>(p, stream);
-        case kOutBf16: return run<false, kUe8m0, false, kOutBf16>(p, stream);
-        case kOutAcc: return run<false, kUe8m0, false, kOutAcc>(p, stream);
-        case kOutAcc2: return run<false, kUe8m0, false, kOutAcc2>(p, stream);
-    }
-    return -1;
+    // bf16 results only: one chain over the whole K rounds f32 results more than
+    // the kernels that split it (2-norm error at K = 5120 1.2e-7 against 0.7e-7;
+    // sums beside the chain every 256 or 512 K 0.8e-7 and 0.7e-7, the latter
+    // still above at some shapes); bf16's own 2^-8 hides it
+    if (omode != kOutBf16 || bfp4 || sbrow) return -1;
+    return smode == kF32s ? run<false, kF32s, false, kOutBf16>(p, stream)
+                          : run<false, kUe8m0, false, kOutBf16>(p, stream);
 }
 
 }  // namespace ws
