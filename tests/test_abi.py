@@ -50,6 +50,27 @@ def test_argument_validation_without_device(lib):
                              4096, 2048, 384, 8, C.c_float(10.0), fake, 16, None) == 1001
 
 
+@pytest.mark.parametrize("rows,dim,inter,experts,top_k", [
+    (8, 4096, 2048, 384, 8),       # few tiles
+    (600, 5120, 2304, 384, 6),     # the stationary pair, padded units
+    (4096, 4096, 2048, 384, 8),    # 96-slot groups
+    (132, 640, 384, 256, 6),       # dim % 256 == 128: the tile-streaming pair
+])
+@pytest.mark.parametrize("native", [False, True])
+def test_prefill_rejects_bad_expert_pointers(rows, dim, inter, experts, top_k, native):
+    """Null or misaligned expert slabs (weights 16 bytes, packed scales 8) are
+    rejected before the first launch, on every body the shape can take."""
+    lib = _lib.load(native=native)
+    fake = 4096  # never dereferenced: validation returns first
+    need = lib.ws_moe_prefill_workspace_size(rows, dim, inter, top_k, experts)
+    for slab in range(6):          # w1, s1, w3, s3, w2, s2
+        for bad in (None, fake + 1, fake + (4 if slab & 1 else 8)):
+            slabs = [fake] * 6
+            slabs[slab] = bad
+            assert lib.ws_moe_prefill(fake, fake, fake, *slabs, fake, rows, dim, inter, experts,
+                                      top_k, C.c_float(10.0), fake, need, None) == 1001, (slab, bad)
+
+
 def test_workspace_sizes(lib):
     n = lib.ws_moe_decode_workspace_size(4096, 2048, 8)
     assert n >= 8 * 2048 + 8 * 64

@@ -1974,7 +1974,9 @@ int ws_moe_prefill(const float *x, const int32_t *topk_idx, const float *topk_w,
         return WS_ERR_INVALID_ARG;
     // every stage's shape limit, checked before the first launch
     if (dim % 128 || inter % 128 || dim > 8192 || inter > 4096) return WS_ERR_SHAPE;
-    if (!w2 || !s2 || !al16(w2) || !al8(s2)) return WS_ERR_INVALID_ARG;
+    if (!w1 || !s1 || !w3 || !s3 || !w2 || !s2) return WS_ERR_INVALID_ARG;
+    if (!al16(w1) || !al16(w3) || !al16(w2) || !al8(s1) || !al8(s3) || !al8(s2))
+        return WS_ERR_INVALID_ARG;
     if (workspace_bytes < ws_moe_prefill_workspace_size(rows, dim, inter, top_k, n_experts) ||
         !al16(workspace))
         return WS_ERR_INVALID_ARG;
