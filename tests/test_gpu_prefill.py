@@ -422,11 +422,24 @@ def test_moe_prefill_rejects_oversized_shapes():
 
 
 @pytest.mark.parametrize("m,E,dim,inter,k", [(40, 64, 1024, 512, 6), (9, 16, 512, 256, 4),
-                                             (40, 256, 640, 384, 6)])
+                                             (40, 256, 640, 384, 6),
+                                             # stationary, padded units: gate/up K parts of 8
+                                             # and 10, 8 and 2, 16 and 24, 0 and 2, 0 and 6,
+                                             # 16 and 16 steps
+                                             (200, 32, 2304, 1152, 6), (300, 24, 1280, 640, 4),
+                                             (100, 64, 5120, 2432, 6), (130, 8, 256, 128, 2),
+                                             (120, 16, 768, 384, 4), (200, 48, 4096, 2176, 4),
+                                             # 96-slot groups: a slice of scratch per workgroup
+                                             # and (few slots, dim 1280 and 2304) per strip
+                                             (1000, 32, 1280, 640, 4), (700, 8, 2304, 1152, 2),
+                                             (600, 16, 768, 384, 4), (4600, 64, 512, 256, 8),
+                                             (4000, 96, 2048, 1024, 6), (2000, 64, 5120, 640, 8)])
 def test_prefill_stages_compose_to_moe_prefill(m, E, dim, inter, k):
     """emit8 -> dispatch -> grouped gate/up -> grouped down (every slot) ->
     combine through the public entry points gives the bits of ws_moe_prefill
-    (which multiplies and writes only the slots that hold routes)."""
+    (which multiplies and writes only the slots that hold routes), on the
+    tile-streaming pair and on the bodies that take its place (not on the
+    stationary pair's whole units: dim and inter in 1024s)."""
     rng = np.random.default_rng(990 + m)
     gen = torch.Generator(device=DEV)
     gen.manual_seed(990 + m)

@@ -1332,11 +1332,22 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
 
     // ---- compute side: the unit being multiplied
     int ri_c = 0, s_c = 0, Tc = 1, t0c = 0, cgc = 0, lo16 = 0, nrc = 0;
+    constexpr bool kParts = MODE == 0 && PAD;  // gate/up sums in two K parts
     // gate/up: the routing weights of the lane's rows r and 16 + r of each
     // tile, loaded when the unit opens (used at its end)
     const es_rsrc lwbuf = es_buf(a.layout_w, (size_t)a.slots * 4);
     float rwf[kTG][2];
+    // the lane, asked for again at each use (as is the unit's column block): what
+    // is held over the stream is spilled beside p0, and a reload from scratch
+    // waits for every load in flight
+    auto lane_at_use = [&]() {
+        int l = lane;
+        if (kParts)
+            __asm__ volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
+        return l;
+    };
     auto open_compute = [&]() {
+        const int r = lane_at_use() & 15;
         const int k = unit_k(ri_c);
         const int v = __builtin_amdgcn_readfirstlane(es_lds_word(&grp_l[k / NCG]));
         nrc = __builtin_amdgcn_readfirstlane(es_lds_word(&nrl_l[k / NCG]));
@@ -1361,6 +1372,14 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
     // operand, so lane (r, g) holds columns 4g .. 4g + 3 of the band for
     // row r of the fragment (four adjacent columns of one row)
     v4f acc[kTG][2][2];
+    // gate/up, PAD: the sums are p0 + p1 over the K parts of grouped_glu_body,
+    // whose bits these are (the shapes that body took alone before): h is
+    // re-quantised, and a longer chain moves more of it by an e4m3 step. p0 waits
+    // in registers of its own; 600 tokens of 384 experts, dim 5120, 1441 us with
+    // one chain, 1459 so.
+    v4f p0[kParts ? kTG : 1][2][2];
+    int kh = 0, kend;
+    if (kParts) k_part8(NS, 1, 2, kh, kend);
     const uint64_t tab = ws_lane_exp2f_tab(lane);
 
     // The scale bytes of four steps (one per step and lane: a word) sit in
@@ -1383,6 +1402,19 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
             for (int j = 0; j < kTG; j++)
 #pragma unroll
                 for (int h = 0; h < 2; h++) acc[j][h][0] = acc[j][h][1] = v4f{0.f, 0.f, 0.f, 0.f};
+        }
+        // kh is whole rounds of eight steps and units begin at steps 0 and 4 of the
+        // iteration; kh = 0: p0 is zero
+        if (kParts && (u & 3) == 0 && s_c == kh) {  // uniform
+#pragma unroll
+            for (int j = 0; j < kTG; j++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        p0[kParts ? j : 0][h][i] = acc[j][h][i];
+                        acc[j][h][i] = v4f{0.f, 0.f, 0.f, 0.f};
+                    }
         }
         if (PAD && s_c >= NS) return;  // uniform: a step past K
         v8bf bq[2][4];
@@ -1444,7 +1476,20 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
         // columns; a row's FP8 1x32 block spans this wave (lanes g = 0..3 of
         // the row's r) and its partner (w ^ 1), which meet in LDS (both
         // tiles' maxima across one barrier)
-        const int col = cgc * 128 + 16 * w + 4 * g;
+        const int ln = lane_at_use(), r = ln & 15, g = ln >> 4;
+        const int col = (kParts ? unit_k(ri_c) % NCG : cgc) * 128 + 16 * w + 4 * g;
+        if (kParts) {
+#pragma unroll
+            for (int j = 0; j < kTG; j++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int i = 0; i < 2; i++)
+#pragma unroll
+                        for (int v = 0; v < 4; v++)
+                            acc[j][h][i][v] = p0[kParts ? j : 0][h][i][v] + acc[j][h][i][v];
+            __builtin_amdgcn_sched_barrier(0);  // p0's registers are free from here
+        }
         float hv[kTG][2][4], m[kTG][2];  // [j][i][v]: tile j, row 16 i + r, column col + v
 #pragma unroll
         for (int j = 0; j < kTG; j++) {
@@ -1619,7 +1664,7 @@ static bool es_fits(int64_t dim, int64_t inter, int64_t tiles) {
 // 12.5 / 32 / 42 routes per expert 889 / 985, 1406 / 1355, 1600 / 1520; 62 and
 // 85 (streaming) 2556 / 1414, 3816 / 2191; dim 5120, inter 2304, top-6 at 62
 // (streaming) 5814 / 2437; 96 experts, dim 2304, inter 1152 at 125 420 / 380.
-// The sums, and so the bits, are the stationary pair's.
+// The sums, and so the bits, are the tile-streaming pair's.
 static bool mt_pays(int64_t rows, int64_t dim, int64_t inter, int64_t slots, int64_t routes,
                     int64_t n_experts, int64_t tiles) {
     if (math_mode() != WS_MATH_EXACT) return false;
@@ -2006,14 +2051,17 @@ int ws_moe_prefill(const float *x, const int32_t *topk_idx, const float *topk_w,
     uint16_t *hbf = (uint16_t *)take(slots * inter * 2);
     // the dispatch and the tokens' quantisation in one launch
     if (n_experts > kMaxExpertsG || routes > (1 << 26) || tiles > (1 << 24)) return WS_ERR_SHAPE;
-    const bool tiled = mt_pays(rows, dim, inter, slots, routes, n_experts, tiles);
+    const bool tiled = mt_pays(rows, dim, inter, slots, routes, n_experts, tiles) &&
+                       moe_tile_parts((size_t)((uint8_t *)xbf - hq), (int)slots, (int)dim, (int)inter) >= 0;
     const bool stationary = !tiled && es_fits(dim, inter, tiles);
     int rc = dispatch_launch(topk_idx, topk_w, order, layout_w, route_pos, tile_expert, cnt, off,
                              psum, ntiles, rows, top_k, tiles, n_experts, x, xq, xs, rows * dim,
                              stream, stationary || tiled ? xbf : nullptr, stationary ? sel : nullptr);
     if (rc) return rc;
     if (tiled) {
-        rc = moe_tile_glu(xbf, order, layout_w, off, cnt, w1, s1, w3, s3, hbf, (int)dim, (int)inter,
+        // its K parts' sums wait in hq .. down, which this step does not use
+        rc = moe_tile_glu(xbf, order, layout_w, off, cnt, w1, s1, w3, s3, hbf, hq,
+                          (size_t)((uint8_t *)xbf - hq), (int)slots, (int)dim, (int)inter,
                           (int)n_experts, (int)top_k, swiglu_limit, stream);
         if (!rc)
             rc = moe_tile_down(hbf, off, cnt, w2, s2, down, (int)dim, (int)inter, (int)n_experts,
@@ -2033,9 +2081,11 @@ int ws_moe_prefill(const float *x, const int32_t *topk_idx, const float *topk_w,
         const bool wide = wide_units(tiles);
         const int grows = dim <= 4096 ? 32 : 16;
         const size_t glds = std::max(es::kLdsAll, g_tile_lds(grows, (int)dim));
+        // dim or inter not whole rounds of the ring
+        const bool parts = dim / 128 % es::kRing || inter / 128 % es::kRing;
 #define WS_GLU_SEL(R, W, P) \
     hipLaunchKernelGGL((glu_select_kernel<R, W, P>), grid, dim3(kGThreads), glds, stream, sel, ea, ga)
-#define WS_GLU_SEL_P(R, W) { if (dim / 128 % es::kRing) WS_GLU_SEL(R, W, true); else WS_GLU_SEL(R, W, false); }
+#define WS_GLU_SEL_P(R, W) { if (parts) WS_GLU_SEL(R, W, true); else WS_GLU_SEL(R, W, false); }
         if (grows == 32) {
             if (wide) WS_GLU_SEL_P(32, 2) else WS_GLU_SEL_P(32, 1)
         } else {

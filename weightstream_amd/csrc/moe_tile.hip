@@ -21,7 +21,14 @@
 //    next 32-K sub-step's weights, as in gemm_tile.hip;
 //  - gate/up: a wave holds the w1 and the w3 rows of 32 intermediate columns,
 //    one FP8 1x32 block per row, so SwiGLU and the re-quantisation need no
-//    other wave.
+//    other wave;
+//  - gate/up sums are p0 + p1 over the two K parts of moe_grouped.hip's
+//    tile-streaming body, whose bits these are: with one chain more of the
+//    re-quantised h moved by an e4m3 step (4096 tokens of 384 experts, dim 4096:
+//    the outputs' 2-norm error against 64 bits 9.3e-5 and 8.0e-5 for two draws,
+//    6.6e-5 and 4.7e-5 so). The registers hold one sum (192 of 256 would go to
+//    two), so p0 waits in scratch memory, 192 KB per workgroup that its next unit
+//    takes again: 2099 -> 2159 us for that prefill.
 // The strips (16 rows) multiplied are those that hold routes: six
 // instantiations, 16 to 96 rows.
 #include "ws_internal.hpp"
@@ -41,6 +48,7 @@ constexpr int kW = kWaves * kNB * 1024;  // weight bytes of a stage
 constexpr int kA = kStrips * 16 * 256;   // A bytes of a stage (bf16, 128 K)
 constexpr int kScale = kWaves * kNB * 256;  // scale bytes of four steps
 constexpr int kMaxE = 1024;
+constexpr int kPartPiece = kNB * 1024;   // bytes of a wave's first sums of one strip
 // LDS: weight stages, two A stages (whole multiples of 1 KB from LDS offset 0: the
 // read addresses are formed by XOR), scale words, the table of groups before
 // each expert
@@ -56,6 +64,8 @@ struct Args {
     const uint8_t *wa, *sa, *wb, *sb;  // gate/up: w1, w3; down: w2
     uint16_t *hbf;                // gate/up out: bf16 h [slots][N]
     float *out;                   // down out: f32 [slots][N]
+    uint8_t *part;                // gate/up: the first K part's sums,
+    int part_by_slot;             // by strip and column, or by workgroup
     int K, N, n_experts, top_k;
     float limit;
 };
@@ -85,28 +95,28 @@ __device__ __forceinline__ void unit(const Args &p, uint8_t *lds, int e, int slo
         }
         ao[q] = arow * (uint32_t)(2 * K) + (uint32_t)(((lane & 15) ^ (row & 15)) * 16);
     }
-    // this wave's bands: gate/up w1, w3 of columns 16h of its 32; down 64 columns
+    // this wave's bands: gate/up w1, w3 of columns 16h of its 32; down 64
+    // columns. N is whole waves' columns, so a wave's are all in it or all past
+    // it (the last ones repeated, unused). One address and the stride to the
+    // next band: eight pointers were spilled to scratch
     const uint32_t l16 = lane * 16, l8 = lane * 8;
     const size_t wmat = (size_t)N * (K / 2), smat = (size_t)packed_fp4_scale_bytes(N, K);
-    const uint8_t *wsrc[kNB], *ssrc[kNB];
     const int c0 = MODE == 0 ? cb * 256 + 32 * w : cb * 512 + 64 * w;  // first column
-#pragma unroll
-    for (int b = 0; b < kNB; b++) {
-        const int rt = min(c0 / 16 + (MODE == 0 ? b >> 1 : b), N / 16 - 1);  // past N: repeated, unused
-        const bool up = MODE == 0 && (b & 1);
-        wsrc[b] = (up ? p.wb : p.wa) + e * wmat + (size_t)rt * n * 1024;
-        ssrc[b] = (up ? p.sb : p.sa) + e * smat + (size_t)rt * ks8 * 512;
-    }
+    const int rt = min(c0 / 16, N / 16 - (MODE == 0 ? 2 : 4));
+    const size_t wat = e * wmat + (size_t)rt * n * 1024, sat = e * smat + (size_t)rt * ks8 * 512;
+    const uint8_t *const wsrc[2] = {p.wa + wat, p.wb + wat}, *const ssrc[2] = {p.sa + sat, p.sb + sat};
     auto issue_a = [&](int q, int s, int buf) {
         dma16(p.a + (size_t)s * 256 + ao[q], lds + kOffA + buf * kA + (w * AL + q) * 1024);
     };
     auto issue_w = [&](int b, int s, int buf) {
-        dma16(wsrc[b] + (size_t)s * 1024 + l16, lds + buf * kW + (w * kNB + b) * 1024);
+        const int m = MODE == 0 ? b & 1 : 0, h = MODE == 0 ? b >> 1 : b;
+        dma16(wsrc[m] + (uint32_t)(h * n + s) * 1024u + l16, lds + buf * kW + (w * kNB + b) * 1024);
     };
     auto issue_scales = [&](int grp) {  // steps 4 grp .. 4 grp + 3
 #pragma unroll
         for (int b = 0; b < kNB; b++)
-            dma4(ssrc[b] + (size_t)(grp >> 1) * 512 + (grp & 1) * 4 + l8,
+            dma4(ssrc[MODE == 0 ? b & 1 : 0] +
+                     (uint32_t)((MODE == 0 ? b >> 1 : b) * ks8 + (grp >> 1)) * 512u + (grp & 1) * 4 + l8,
                  lds + kOffS + (w * kNB + b) * 256);
     };
     issue_scales(0);
@@ -172,8 +182,32 @@ __device__ __forceinline__ void unit(const Args &p, uint8_t *lds, int e, int slo
     settle_w(0);
     seq([&](auto pc) { conv_b(Z{}, pc); }, WS_SEQ(16, p));
 
+    // gate/up: the step at which the second K part begins (0: it is the whole),
+    // and where the first one's sums of strip i wait, 16 bytes per lane and band
+    int kh = 0, kend;
+    if (MODE == 0) k_part8(n, 1, 2, kh, kend);
+    if (c0 >= N) kh = 0;  // uniform: a wave past the last column keeps nothing
+    const uint32_t pstride = (uint32_t)(MODE == 0 && p.part_by_slot ? N / 32 : kWaves) * kPartPiece;
+    auto part_at = [&]() {  // strip 0's; formed at each use: nothing is held over the loop
+        int sl = slot0;
+        __asm__ volatile("" : "+s"(sl));
+        const size_t at = p.part_by_slot ? (size_t)(sl / 16) * (N / 32) + c0 / 32
+                                         : (size_t)(blockIdx.x * kStrips) * kWaves + w;
+        return p.part + at * kPartPiece + l16;
+    };
+
     int w1 = 1;  // (s + 1) % kNW
     for (int s = 0; s < n; s++) {
+        if (MODE == 0 && s == kh && kh > 0) {  // uniform
+            uint8_t *const pt = part_at();
+#pragma unroll
+            for (int i = 0; i < MF; i++)
+#pragma unroll
+                for (int b = 0; b < kNB; b++) {
+                    *(v4f *)(pt + i * (size_t)pstride + b * 1024) = acc[i][b];
+                    acc[i][b] = v4f{0.f, 0.f, 0.f, 0.f};
+                }
+        }
         raw_barrier();  // step s is in LDS; the other stage has been read by every wave
         const uint32_t a0 = ra + (s & 1) * kA;
         const uint32_t stn = w1 * kW;
@@ -237,6 +271,20 @@ __device__ __forceinline__ void unit(const Args &p, uint8_t *lds, int e, int slo
         }, WS_SEQ(T, t));
         w1 = w2;
     }
+    // the first K part's sums, loaded two strips ahead of their use
+    v4f p0[2][kNB];
+    const uint8_t *const pt = part_at();
+    auto load_p0 = [&](int i) {
+#pragma unroll
+        for (int b = 0; b < kNB; b++) {
+            p0[i & 1][b] = v4f{0.f, 0.f, 0.f, 0.f};
+            if (kh > 0) p0[i & 1][b] = *(const v4f *)(pt + i * (size_t)pstride + b * 1024);
+        }
+    };
+    if (MODE == 0) {
+        load_p0(0);
+        if (MF > 1) load_p0(1);
+    }
     wait_vm<0>();  // the repeated copies still write this workgroup's LDS
 
     // ---- store: columns 4g .. 4g + 3 of a band, row r of a strip
@@ -265,11 +313,17 @@ __device__ __forceinline__ void unit(const Args &p, uint8_t *lds, int e, int slo
         if (16 * i >= rows) continue;  // uniform
         const int row = 16 * i + r;
         float hv[2][4], m = 0.0f;
+        v4f sum[kNB];
+#pragma unroll
+        for (int b = 0; b < kNB; b++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) sum[b][v] = p0[i & 1][b][v] + acc[i][b][v];
+        if (i + 2 < MF) load_p0(i + 2);
 #pragma unroll
         for (int h = 0; h < 2; h++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                float gv = acc[i][2 * h][v], uv = acc[i][2 * h + 1][v];
+                float gv = sum[2 * h][v], uv = sum[2 * h + 1][v];
                 if (p.limit > 0.0f) {
                     uv = rclamp(uv, -p.limit, p.limit);
                     gv = fminf(gv, p.limit);
@@ -370,12 +424,24 @@ __global__ __launch_bounds__(kThreads) void moe_tile_kernel(const Args p) {
 
 }  // namespace mt
 
+// 0: no scratch needed (one K part), 1: a slice per workgroup (the slices stay
+// in the caches), 2: where those do not fit (few slots), a piece per strip and
+// 32 columns; -1: neither fits.
+int moe_tile_parts(size_t part_bytes, int slots, int dim, int inter) {
+    if ((dim / 128 + kU - 1) / kU < 2) return 0;
+    if ((size_t)cu_count() * mt::kStrips * mt::kWaves * mt::kPartPiece <= part_bytes) return 1;
+    return (size_t)(slots / 16) * (inter / 32) * mt::kPartPiece <= part_bytes ? 2 : -1;
+}
+
 int moe_tile_glu(const uint16_t *xbf, const int32_t *order, const float *layout_w,
                  const int32_t *exp_off, const int32_t *exp_cnt, const uint8_t *w1,
-                 const uint8_t *s1, const uint8_t *w3, const uint8_t *s3, uint16_t *hbf, int dim,
-                 int inter, int n_experts, int top_k, float limit, hipStream_t stream) {
+                 const uint8_t *s1, const uint8_t *w3, const uint8_t *s3, uint16_t *hbf,
+                 uint8_t *part, size_t part_bytes, int slots, int dim, int inter, int n_experts,
+                 int top_k, float limit, hipStream_t stream) {
+    const int mode = moe_tile_parts(part_bytes, slots, dim, inter);
+    if (mode < 0) return WS_ERR_SHAPE;
     const mt::Args p{(const uint8_t *)xbf, order, layout_w, exp_off, exp_cnt, w1, s1, w3, s3, hbf,
-                     nullptr, dim, inter, n_experts, top_k, limit};
+                     nullptr, part, mode == 2, dim, inter, n_experts, top_k, limit};
     hipLaunchKernelGGL(mt::moe_tile_kernel<0>, dim3((unsigned)cu_count()), dim3(mt::kThreads),
                        mt::kLds, stream, p);
     return launch_status();
@@ -385,7 +451,7 @@ int moe_tile_down(const uint16_t *hbf, const int32_t *exp_off, const int32_t *ex
                   const uint8_t *w2, const uint8_t *s2, float *out, int dim, int inter,
                   int n_experts, hipStream_t stream) {
     const mt::Args p{(const uint8_t *)hbf, nullptr, nullptr, exp_off, exp_cnt, w2, s2, nullptr,
-                     nullptr, nullptr, out, inter, dim, n_experts, 1, 0.0f};
+                     nullptr, nullptr, out, nullptr, 0, inter, dim, n_experts, 1, 0.0f};
     hipLaunchKernelGGL(mt::moe_tile_kernel<1>, dim3((unsigned)cu_count()), dim3(mt::kThreads),
                        mt::kLds, stream, p);
     return launch_status();

@@ -52,11 +52,15 @@ int tile_gemm(bool bfp4, int smode, bool sbrow, int omode, const uint8_t *a, con
               const uint8_t *b, const void *sb, void *out, const float *aux, int64_t m, int64_t n,
               int64_t k, hipStream_t stream);
 // moe_tile.hip: the grouped gate/up (bf16 h out) and down steps over 96-slot
-// groups, exact math; offsets and counts are the dispatch's.
+// groups, exact math; offsets and counts are the dispatch's. part: scratch of
+// part_bytes for the gate/up sums of the first K part; moe_tile_parts says how
+// it is used, -1 where it is too small for the shape.
+int moe_tile_parts(size_t part_bytes, int slots, int dim, int inter);
 int moe_tile_glu(const uint16_t *xbf, const int32_t *order, const float *layout_w,
                  const int32_t *exp_off, const int32_t *exp_cnt, const uint8_t *w1,
-                 const uint8_t *s1, const uint8_t *w3, const uint8_t *s3, uint16_t *hbf, int dim,
-                 int inter, int n_experts, int top_k, float limit, hipStream_t stream);
+                 const uint8_t *s1, const uint8_t *w3, const uint8_t *s3, uint16_t *hbf,
+                 uint8_t *part, size_t part_bytes, int slots, int dim, int inter, int n_experts,
+                 int top_k, float limit, hipStream_t stream);
 int moe_tile_down(const uint16_t *hbf, const int32_t *exp_off, const int32_t *exp_cnt,
                   const uint8_t *w2, const uint8_t *s2, float *out, int dim, int inter,
                   int n_experts, hipStream_t stream);
