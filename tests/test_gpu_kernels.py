@@ -114,11 +114,16 @@ def test_weight_quant_bit_exact():
 
 
 @pytest.mark.parametrize("n,skew", [(32, 0), (1024, 0), (2048 + 32, 0), (3 * 2048 - 32, 0),
-                                    (32, 1), (2048 + 96, 1)])
+                                    (32, 1), (2048 + 96, 1),
+                                    (384 * 1024 - 32, 0), (384 * 1024, 0), (458752 - 128, 0),
+                                    (458752, 0), (768 * 1024 - 32, 0), (768 * 1024, 0),
+                                    (768 * 1024 + 2048 + 128, 0), (768 * 1024 + 3 * 2048 - 32, 0),
+                                    (768 * 1024 + 128, 1)])
 def test_act_quant_edges_and_unaligned(n, skew):
     """The four-values-per-lane kernels at the edges of their 2048-value
-    workgroups, and the one-value kernels that unaligned operands (skew floats
-    and bytes off) take: bit-exact."""
+    workgroups, and the one- and two-value kernels that fewer values (384 K for
+    bytes, 768 K in place, 448 K with f32 scales) and unaligned operands (skew
+    floats and bytes off) take: bit-exact."""
     rng = np.random.default_rng(103 + n)
     x = _wide_range_acts(rng, max(n, 128))[:n].copy()
     q_ref, s_ref = O.fp8_act_emit(x)
@@ -149,11 +154,14 @@ def test_act_quant_edges_and_unaligned(n, skew):
 
 
 @pytest.mark.parametrize("rows,cols,skew", [(1, 32, 0), (33, 160, 0), (31, 96, 0), (64, 384, 0),
-                                            (33, 160, 1)])
+                                            (33, 160, 1),
+                                            (255, 1056, 0), (256, 1056, 0), (1023, 1024, 0),
+                                            (1025, 1056, 0), (1025, 1056, 1)])
 def test_weight_quant_edges_and_unaligned(rows, cols, skew):
-    """The vectorised weight encoders at ragged rows and columns, with FP4
-    values on and beside every rounding threshold, and the fallback for
-    unaligned operands: bit-exact."""
+    """The vectorised weight encoders (from 256 K values in FP4, 1 M in FP8) at
+    ragged rows and columns, with FP4 values on and beside every rounding
+    threshold, and the kernels for fewer values and unaligned operands:
+    bit-exact."""
     rng = np.random.default_rng(104 + rows + cols)
     w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
     edges = np.array([0.25, 0.75, 1.0, 1.25, 1.75, 2.5, 3.5, 5.0, 6.0], np.float32)
@@ -175,6 +183,64 @@ def test_weight_quant_edges_and_unaligned(rows, cols, skew):
     L.weight_quant_fp8(dw, q8, s8, rows, cols)
     q8r, s8r = O.weight_quant_fp8(w)
     assert np.array_equal(host(q8), q8r.ravel()) and np.array_equal(host(s8), s8r.ravel())
+
+
+def test_weight_quant_nonfinite_same_on_both_kernels():
+    """Blocks with infinities, NaN, nothing else, and FLT_MAX: the vectorised
+    encoders give the bytes of the general ones (which unaligned operands
+    take)."""
+    rows, cols = 1024, 1056
+    rng = np.random.default_rng(105)
+    w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
+    big = np.finfo(np.float32).max
+    w[0, 5], w[40, 70], w[41, 71], w[100, 1040] = np.inf, -np.inf, np.nan, np.nan
+    w[200, 64:96] = np.inf
+    w[224:256, 96:128] = np.nan
+    w[300, 128:160] = np.nan
+    w[400, 1000], w[401, 1001], w[500, 32:64] = big, -big, big
+    w[600, 0:32] = 1e-42
+    announce("weight_quant nonfinite %dx%d on both kernels" % (rows, cols))
+    out = []
+    for skew in (0, 1):
+        dw = torch.empty(rows * cols + skew, device=DEV)[skew:]
+        dw.copy_(dev(w.ravel()))
+        q4 = torch.empty(rows * cols // 2, dtype=torch.uint8, device=DEV)
+        q8 = torch.empty(rows * cols, dtype=torch.uint8, device=DEV)
+        s4 = torch.empty(rows * cols // 32, dtype=torch.uint8, device=DEV)
+        s8 = torch.empty(rows // 32 * (cols // 32), dtype=torch.uint8, device=DEV)
+        L.weight_quant_fp4(dw, q4, s4, rows, cols)
+        L.weight_quant_fp8(dw, q8, s8, rows, cols)
+        out.append([host(t) for t in (q4, s4, q8, s8)])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("rows,cols", [(16, 128), (48, 1024), (2064, 1024), (32, 1152),
+                                       (2048, 2048), (2064, 2048), (272, 5120), (16, 2944)])
+def test_prepack_layout(rows, cols):
+    """The packed layout's definition, in numpy, for the relayout by chunks
+    (whole 8-step scale groups, small or one group long) and by waves; padding
+    scale bytes are 127."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(rows + cols)
+    announce("prepack %dx%d" % (rows, cols))
+    w = torch.randint(0, 256, (rows, cols // 2), dtype=torch.uint8, device=DEV, generator=gen)
+    s = torch.randint(0, 256, (rows, cols // 32), dtype=torch.uint8, device=DEV, generator=gen)
+    for skew in (0, 1):
+        pw = torch.full((rows * cols // 2 + 16,), 0xA5, dtype=torch.uint8, device=DEV)
+        n = L.packed_fp4_scale_bytes(rows, cols)
+        ps = torch.full((n + skew + 16,), 0xA5, dtype=torch.uint8, device=DEV)
+        L.prepack_fp4(w, s, rows, cols, pw, ps[skew:])
+        ksn = cols // 128
+        # [band][step][16 g + r][16 bytes]: row 16 band + r, chunk 4 step + g
+        want = host(w).reshape(rows // 16, 16, ksn, 4, 16).transpose(0, 2, 3, 1, 4)
+        sc = np.full((rows // 16, (ksn + 7) // 8 * 8, 4, 16), 127, np.uint8)
+        sc[:, :ksn] = host(s).reshape(rows // 16, 16, ksn, 4).transpose(0, 2, 3, 1)
+        # [band][group][16 g + r][step of the group]
+        sc = sc.reshape(rows // 16, -1, 8, 64).transpose(0, 1, 3, 2)
+        got, gs = host(pw), host(ps)[skew:]
+        assert np.array_equal(got[:-16], want.ravel()) and (got[-16:] == 0xA5).all()
+        assert np.array_equal(gs[:n], sc.ravel()) and (gs[n:] == 0xA5).all()
 
 
 def _quantised_case(rng, m, n, k, fp4):

@@ -44,9 +44,9 @@ def _nonfinite_acts(rng, nblk, block=32):
     return x
 
 
-def test_emit8_snap8_nonfinite_blocks():
+@pytest.mark.parametrize("n", [32 * 64, 32 * 24576])   # one and four values per lane
+def test_emit8_snap8_nonfinite_blocks(n):
     rng = np.random.default_rng(900)
-    n = 32 * 64
     x = _nonfinite_acts(rng, n // 32)
     q_ref, s_ref = O.fp8_act_emit(x)
     assert q_ref[3] == 0xFF and s_ref[0] == 0xFF     # the rule this file states
@@ -74,9 +74,9 @@ def test_emit8_snap8_nonfinite_blocks():
     assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
 
 
-def test_act_quant_f32s_nonfinite_blocks():
+@pytest.mark.parametrize("m,k", [(2, 1024), (512, 1024)])   # two and four values per lane
+def test_act_quant_f32s_nonfinite_blocks(m, k):
     rng = np.random.default_rng(901)
-    m, k = 2, 1024
     x = _nonfinite_acts(rng, m * k // 128, 128).reshape(m, k)
     aq_ref, as_ref = O.act_quant_f32s(x, 128)
     announce("act_quant_f32s nonfinite m=%d k=%d" % (m, k))
@@ -87,9 +87,9 @@ def test_act_quant_f32s_nonfinite_blocks():
     assert np.array_equal(host(as_).view(np.uint32).ravel(), as_ref.view(np.uint32).ravel())
 
 
-def test_weight_quant_fp8_nonfinite_blocks():
+@pytest.mark.parametrize("rows,cols", [(96, 128), (1024, 1024)])   # one and four blocks per workgroup
+def test_weight_quant_fp8_nonfinite_blocks(rows, cols):
     rng = np.random.default_rng(902)
-    rows, cols = 96, 128
     w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
     w[0, 0] = np.inf
     w[40, 70] = -np.inf

@@ -82,17 +82,38 @@ __global__ __launch_bounds__(256) void pack_scale_words_kernel(const uint8_t *sr
              ((uint32_t)p[3] << 24);
 }
 
-// f32-scale activation quant: half a wave per 1x128 block, four consecutive
-// values per lane (one float4 load and one 4-byte store when VEC: x 16-byte
-// and q 4-byte aligned).
-template <bool VEC>
+// f32-scale activation quant: one wave per 1x128 block, two values per lane.
 __global__ __launch_bounds__(256) void act_quant_f32s_kernel(const float *x, uint8_t *q, float *s,
                                                              int64_t blocks) {
+    int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (b >= blocks) return;  // whole wave exits together
+    int l = threadIdx.x & 63;
+    const float *v = x + b * 128;
+    float x0 = v[l], x1 = v[l + 64];
+    float amax = fmaxf(__builtin_fabsf(x0), __builtin_fabsf(x1));
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+    if (!(amax >= 1e-4f)) amax = 1e-4f;  // an all-NaN block too, as the reference's `a > amax` scan
+    float sc = amax / 448.0f;
+    // inf / inf (a block holding an infinity) is the host's invalid-operation
+    // NaN, sign bit set on x86: byte 0xFF, as block_byte
+    const bool inf_blk = sc == __builtin_inff();
+    const uint32_t q0 = f32_to_e4m3(rclamp(x0 / sc, -448.0f, 448.0f));
+    const uint32_t q1 = f32_to_e4m3(rclamp(x1 / sc, -448.0f, 448.0f));
+    q[b * 128 + l] = (uint8_t)(inf_blk && __builtin_fabsf(x0) == sc ? 0xFFu : q0);
+    q[b * 128 + l + 64] = (uint8_t)(inf_blk && __builtin_fabsf(x1) == sc ? 0xFFu : q1);
+    if (l == 0) s[b] = sc;
+}
+
+// The same with half a wave per block and four consecutive values per lane (one
+// float4 load and one 4-byte store): 21.0 M values 39.3 -> 30.9 us. Taken for
+// many values (see the launch), x 16-byte and q 4-byte aligned.
+__global__ __launch_bounds__(256) void act_quant_f32s4_kernel(const float *x, uint8_t *q, float *s,
+                                                              int64_t blocks) {
     const int64_t b = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
     const bool live = b < blocks;
     const int l = threadIdx.x & 31;
-    const float *v = x + (live ? b : 0) * 128 + 4 * l;
-    const float4 f = VEC ? *(const float4 *)v : float4{v[0], v[1], v[2], v[3]};
+    const float4 f = *(const float4 *)(x + (live ? b : 0) * 128 + 4 * l);
     float amax = half_wave_max(fmaxf(fmaxf(__builtin_fabsf(f.x), __builtin_fabsf(f.y)),
                                      fmaxf(__builtin_fabsf(f.z), __builtin_fabsf(f.w))));
     if (!(amax >= 1e-4f)) amax = 1e-4f;  // an all-NaN block too, as the reference's `a > amax` scan
@@ -106,13 +127,7 @@ __global__ __launch_bounds__(256) void act_quant_f32s_kernel(const float *x, uin
     };
     const uint32_t w = byte(f.x) | (byte(f.y) << 8) | (byte(f.z) << 16) | (byte(f.w) << 24);
     if (!live) return;
-    uint8_t *o = q + b * 128 + 4 * l;
-    if (VEC) {
-        *(uint32_t *)o = w;
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; j++) o[j] = (uint8_t)(w >> (8 * j));
-    }
+    *(uint32_t *)(q + b * 128 + 4 * l) = w;
     if (l == 0) s[b] = sc;
 }
 
@@ -346,8 +361,13 @@ int ws_expf_probe(uint32_t lo, uint32_t n, uint32_t *out, ws_stream_t stream) {
 static int act_quant_launch(int mode, float *xio, const float *x, uint8_t *q, uint8_t *s,
                             int64_t n, int64_t packed, ws_stream_t stream) {
     if (n <= 0 || n % 32) return WS_ERR_SHAPE;
-    // four values per lane when the loads and stores are aligned for it
-    if (((uintptr_t)(mode == 1 ? xio : x) & 15) == 0 && ((uintptr_t)q & 3) == 0) {
+    // four values per lane and two passes when the loads and stores are aligned
+    // for it and the workgroups fill the chip; below, a value per lane ends
+    // sooner. us, one value / four: bytes 27 x 8192 values 2.48 / 2.74, 384 K
+    // 2.90 / 2.84, 1 M 4.25 / 3.13; in place 27 x 8192 2.58 / 3.33, 640 K 3.66 /
+    // 3.88, 768 K 3.88 / 3.85, 1 M 4.58 / 4.03.
+    if (((uintptr_t)(mode == 1 ? xio : x) & 15) == 0 && ((uintptr_t)q & 3) == 0 &&
+        n >= (mode == 1 ? 768 : 384) * 1024) {
         const dim3 grid((unsigned)((n + 1024 * kAqPasses - 1) / (1024 * kAqPasses)));
         if (mode == 1)
             hipLaunchKernelGGL(act_quant4_kernel<1>, grid, dim3(256), 0, stream, xio, x, q, s, n, packed);
@@ -394,11 +414,14 @@ int ws_act_quant_f32s(const float *x, uint8_t *q, float *s, int64_t m, int64_t k
     if (!x || !q || !s) return WS_ERR_INVALID_ARG;
     if (m <= 0 || k <= 0 || k % 128) return WS_ERR_SHAPE;
     int64_t blocks = m * (k / 128);
-    const dim3 grid((unsigned)((blocks + 7) / 8));
-    if (((uintptr_t)x & 15) == 0 && ((uintptr_t)q & 3) == 0)
-        hipLaunchKernelGGL(act_quant_f32s_kernel<true>, grid, dim3(256), 0, stream, x, q, s, blocks);
+    // us, two values per lane / four: 27 x 4096 values 2.17 / 2.32, 384 K 2.49 /
+    // 2.63, 448 K 2.80 / 2.75, 1 M 3.63 / 3.29
+    if (((uintptr_t)x & 15) == 0 && ((uintptr_t)q & 3) == 0 && blocks >= 448 * 8)
+        hipLaunchKernelGGL(act_quant_f32s4_kernel, dim3((unsigned)((blocks + 7) / 8)), dim3(256), 0,
+                           stream, x, q, s, blocks);
     else
-        hipLaunchKernelGGL(act_quant_f32s_kernel<false>, grid, dim3(256), 0, stream, x, q, s, blocks);
+        hipLaunchKernelGGL(act_quant_f32s_kernel, dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0,
+                           stream, x, q, s, blocks);
     return launch_status();
 }
 
@@ -407,7 +430,9 @@ int ws_weight_quant_fp4(const float *w, uint8_t *q, uint8_t *s, int64_t rows, in
     if (!w || !q || !s) return WS_ERR_INVALID_ARG;
     if (rows <= 0 || cols <= 0 || cols % 32) return WS_ERR_SHAPE;
     int64_t n = rows * cols;
-    if (((uintptr_t)w & 15) == 0 && ((uintptr_t)q & 3) == 0) {
+    // us, one value per lane / eight: 128 x 512 2.29 / 2.41, 128 x 1024 2.39 /
+    // 2.42, 256 x 1024 2.54 / 2.46, 512 x 1024 3.21 / 2.52
+    if (((uintptr_t)w & 15) == 0 && ((uintptr_t)q & 3) == 0 && n >= 256 * 1024) {
         hipLaunchKernelGGL(weight_quant_fp4x8_kernel, dim3((unsigned)((n + 2047) / 2048)), dim3(256),
                            0, stream, w, q, s, n);
         return launch_status();
@@ -422,7 +447,11 @@ int ws_weight_quant_fp8(const float *w, uint8_t *q, uint8_t *s, int64_t rows, in
     if (!w || !q || !s) return WS_ERR_INVALID_ARG;
     if (rows <= 0 || cols <= 0 || cols % 32 || rows > (1 << 24) || cols > (1 << 24))
         return WS_ERR_SHAPE;
-    if (((uintptr_t)w & 15) == 0 && ((uintptr_t)q & 3) == 0) {
+    // us, one block per workgroup / four: 512 x 1024 3.29 / 3.75, 768 x 1024 3.61 /
+    // 3.77, 1024 x 1024 4.06 / 3.79, 2048 x 1024 5.97 / 4.66; with one or two blocks
+    // across half the workgroup idles: 32768 x 64 6.07 / 6.58, 16384 x 96 5.13 / 4.55
+    if (((uintptr_t)w & 15) == 0 && ((uintptr_t)q & 3) == 0 && cols >= 96 &&
+        rows * cols >= 1024 * 1024) {
         hipLaunchKernelGGL(weight_quant_fp8x4_kernel,
                            dim3((unsigned)((cols + 127) / 128), (unsigned)((rows + 31) / 32)),
                            dim3(256), 0, stream, w, q, s, (int)rows, (int)cols);
