@@ -286,11 +286,16 @@ def test_device_e4m3_and_activation_scale_equal_oracle_on_every_input():
 
 @pytest.mark.parametrize("m,E,dim,bf16", [(700, 150, 320, False), (700, 150, 320, True),
                                           (1030, 200, 128, False), (2100, 300, 64, True),
-                                          (4100, 300, 192, False)])
+                                          (4100, 300, 192, False),
+                                          # few experts: blocks at dim 256, lanes at 320
+                                          (12290, 8, 256, False), (12290, 8, 320, True),
+                                          # lanes in f32, blocks in bf16
+                                          (4099, 33, 512, False), (4099, 33, 512, True)])
 def test_gate_logits_many_tokens_bit_exact(m, E, dim, bf16):
     """One expert and 1, 2 or 4 tokens per lane (98304 or more chains): ragged
     expert blocks and token groups, an odd number of 64-element chunks, f32 and
-    bf16 weights; the sequential f32 dots of the oracle bit for bit."""
+    bf16 weights; and the 8 x 8 blocks that as many chains of few experts keep.
+    The sequential f32 dots of the oracle bit for bit."""
     gen = torch.Generator(device=DEV).manual_seed(m + E)
     x = torch.randn((m, dim), device=DEV, generator=gen)
     w = torch.randn((E, dim), device=DEV, generator=gen) * 0.02

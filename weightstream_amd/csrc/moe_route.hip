@@ -519,6 +519,18 @@ __global__ __launch_bounds__(256) void math_probe_kernel(int fn, uint32_t lo, ui
     if (i < n) out[i] = a == b ? a : 0x7fbadbadu;
 }
 
+// Whether one expert and T tokens per lane beat the 8 x 8 blocks. Both times go
+// with dim; at 4096 the blocks take 49 ns each (bf16 weights 43) in rounds of two
+// workgroups per CU, the lanes 15.6 ns per wave of 64 experts, few or many of them
+// real, and 42 us (53) of chain latency. 8192 tokens, f32, us, blocks / lanes: 16 experts
+// 104 / 174, 24 153 / 176, 32 203 / 176, 48 304 / 179; bf16 24 133 / 182, 32 190 /
+// 183, 48 260 / 186; 12288 tokens of 8 experts 78 / 219.
+static bool gate_many_pays(int64_t m, int64_t n_experts, int bf16) {
+    const int64_t round = 2 * cu_count(), waves = m * ((n_experts + 63) / 64);
+    const int64_t blocks = (((m + 7) / 8) * ((n_experts + 7) / 8) + round - 1) / round * round;
+    return bf16 ? 276 * blocks > 100 * (waves + 3400) : 317 * blocks > 100 * (waves + 2700);
+}
+
 static int gate_logits_launch(const float *x, const void *gw, int bf16, float *logits, int64_t m,
                               int64_t dim, int64_t n_experts, hipStream_t stream) {
     if (!x || !gw || !logits) return WS_ERR_INVALID_ARG;
@@ -526,9 +538,11 @@ static int gate_logits_launch(const float *x, const void *gw, int bf16, float *l
     if (dim % 8 || m > 65535 || n_experts > (1 << 20)) return WS_ERR_SHAPE;
     // many chains: one expert and T tokens per lane; T grows with the waves that
     // leaves per SIMD (m tokens x blocks of 64 experts). 384 experts, dim 4096, f32
-    // weights, against the 8 x 8 blocks below, us: 128 tokens 52 / 67, 256 79 /
-    // 67, 1024 300 / 141, 2048 595 / 217, 4096 1182 / 394; bf16 1024 256 / 153.
-    if (dim % 64 == 0 && m * n_experts >= 96 * 1024 && ((uintptr_t)gw & 15) == 0) {
+    // weights, against the 8 x 8 blocks below, us: 128 tokens 52 / 67, 256 77 /
+    // 73, 1024 306 / 144, 2048 605 / 238, 4096 1185 / 420; bf16 256 67 / 86, 512 130
+    // / 99, 4096 1007 / 424. See gate_many_pays.
+    if (dim % 64 == 0 && m * n_experts >= 96 * 1024 && ((uintptr_t)gw & 15) == 0 &&
+        (dim % kGC != 0 || gate_many_pays(m, n_experts, bf16))) {
         const int64_t waves = m * ((n_experts + 63) / 64);
         if (waves <= 3072) gate_many_launch<1, 4, 64>(x, gw, bf16, logits, m, dim, n_experts, stream);
         else if (waves <= 8192) gate_many_launch<2, 4, 64>(x, gw, bf16, logits, m, dim, n_experts, stream);
