@@ -592,16 +592,21 @@ def test_line_gemm_ragged_rows_vs_fp64_dequant(m, n, k, native):
 
 
 @pytest.mark.parametrize("m,n,k", [(129, 400, 128), (200, 528, 256), (777, 4608, 384),
-                                   (2000, 4096, 512), (4090, 4080, 640), (65, 4096, 1152)])
+                                   (2000, 4096, 512), (4090, 4080, 640), (65, 4096, 1152),
+                                   (65, 4112, 1152), (775, 4592, 640)])
 def test_tile_gemm_edges_vs_fp64_dequant(m, n, k):
-    """The whole-K tile kernel in each of its tilings (64 x 128, 128 x 128,
-    128 x 256, 256 x 256) with ragged rows, columns and step counts (1, 2, 3, 4,
-    5 and 9 steps, so that scale groups of four end anywhere), every weight
-    format and epilogue. f32 sums of at most 36 MFMAs: each rounding is at most
-    2^-24 of a partial sum, so the 2-norm error stays under sqrt(36) 2^-24 =
-    3.6e-7; The tiles serve the bf16 output; the f32 and accumulating ones take other
-    kernels whose sums differ in order. Each is within 40 roundings of at most
-    2^-23 of the sum of magnitudes; bf16 adds 2^-8 and the accumulation 2^-23."""
+    """The GEMMs above 64 rows with ragged rows, columns and step counts (1, 2, 3,
+    4, 5 and 9 steps, so that scale groups of four end anywhere), every weight
+    format and output. bf16 results take the whole-K tile kernel (but for 65 x
+    4096, whose columns make one round of 32-column strips), by its rule in 64 x
+    128 tiles (129, 200 and 65 rows), 128 x 128 (777, 775), 128 x 256 (2000; f32
+    scales also 4090) and 256 x 256 (4090); f32 results, FP4 and the accumulating
+    output take the pipeline or the strips.
+
+    f32 sums of at most 36 MFMAs: each rounding is at most 2^-24 of a partial sum,
+    so the 2-norm error stays under sqrt(36) 2^-24 = 3.6e-7. Per value, an MFMA,
+    an f32-scale fma and the scales' product each err by at most 2^-23 of the sum
+    of magnitudes, and bf16 adds 2^-8 of the value."""
     gen = torch.Generator(device=DEV)
     gen.manual_seed(m + n + k)
     announce("tile gemm m=%d n=%d k=%d" % (m, n, k))
@@ -636,9 +641,17 @@ def test_tile_gemm_edges_vs_fp64_dequant(m, n, k):
         print("[tile %s %dx%dx%d] rel 2-norm err %.3g" % (what, m, n, k, err))
         assert err <= 3.6e-7, (what, err)
 
+    def close_bf16(got, want, mags, what):
+        roundings = k // 32 + k // 128 + 2
+        bound = 2.0 ** -8 * want.abs() + roundings * 2.0 ** -23 * mags
+        over = ((got.double() - want).abs() / bound).max()
+        print("[tile %s %dx%dx%d] %.3g of the bound" % (what, m, n, k, float(over)))
+        assert over <= 1, (what, float(over))
+
     out = run(lambda o: L.fp8_gemm(aq, as_, wq, ws, o, m, n, k))
     close(out, da @ dw.T, "fp8")
     ob = run(lambda o: L.fp8_gemm_bf16(aq, as_, wq, ws, o, m, n, k), torch.bfloat16)
+    close_bf16(ob, da @ dw.T, da.abs() @ dw.abs().T, "fp8 bf16")
     if m > 128:  # at most 128 rows ws_fp8_gemm may take the line kernel for both
         slack = 2 * 40 * 2.0 ** -23 * (da.abs() @ dw.abs().T)
         assert ((ob.double() - out.double()).abs() <= 2.0 ** -8 * out.double().abs() + 1.01 * slack).all()
@@ -649,9 +662,11 @@ def test_tile_gemm_edges_vs_fp64_dequant(m, n, k):
     af = torch.rand((m, k // 128), device=DEV, generator=gen) * 0.01 + 1e-3
     wf = torch.rand(((n + 127) // 128, k // 128), device=DEV, generator=gen) * 1e-4 + 1e-5
     fout = run(lambda o: L.fp8_gemm_f32s(aq, af, wq, wf, o, m, n, k))
-    want = ((codes * af.double().repeat_interleave(128, 1))
-            @ (table[wq.long()] * wf.double().repeat_interleave(128, 0)[:n].repeat_interleave(128, 1)).T)
-    close(fout, want, "f32s")
+    fa = codes * af.double().repeat_interleave(128, 1)
+    fw = table[wq.long()] * wf.double().repeat_interleave(128, 0)[:n].repeat_interleave(128, 1)
+    close(fout, fa @ fw.T, "f32s")
+    fob = run(lambda o: L.fp8_gemm_f32s(aq, af, wq, wf, o, m, n, k, out_bf16=True), torch.bfloat16)
+    close_bf16(fob, fa @ fw.T, fa.abs() @ fw.abs().T, "f32s bf16")
     lut = torch.tensor([O.fp4_value(i) for i in range(16)], dtype=torch.float64, device=DEV)
     d4 = torch.stack((lut[(w4 & 15).long()], lut[(w4 >> 4).long()]), -1).view(n, k)
     got = run(lambda o: L.fp4_gemm(aq, as_, w4, s4, o, m, n, k))
@@ -659,14 +674,14 @@ def test_tile_gemm_edges_vs_fp64_dequant(m, n, k):
 
 
 @pytest.mark.parametrize("m", [65, 130, 520])
-def test_tile_gemm_packed_scale_table(m):
-    """ws_fp8_gemm_tl above 64 rows: per-row weight scale words, each row with
-    scales of its own, against f64."""
+def test_packed_scale_table_above_64_rows(m):
+    """ws_fp8_gemm_tl above 64 rows (the column-strip kernel): per-row weight
+    scale words, each row with scales of its own, against f64."""
     kind = L.TL_QB
     n, k = L.tl_gemm_shape(kind)
     gen = torch.Generator(device=DEV)
     gen.manual_seed(m)
-    announce("tile gemm tl m=%d" % m)
+    announce("packed scale table m=%d" % m)
     x = torch.randn((m, k), device=DEV, generator=gen)
     aq = torch.empty((m, k), dtype=torch.uint8, device=DEV)
     as_ = torch.empty((m, k // 32), dtype=torch.uint8, device=DEV)
