@@ -1133,15 +1133,10 @@ static int gemm_dispatch(const uint8_t *a, const void *sa, const uint8_t *b, con
         return WS_ERR_INVALID_ARG;
     int M = (int)m, N = (int)n, K = (int)k;
     const SkWorkspace wsp = sk_ws(stream);
-    const bool exact = math_mode() == WS_MATH_EXACT;
-    auto tiled = [&]() {
-        return tile_gemm(BFP4, SMODE, !BFP4 && sb_div != 32, OMODE, a, sa, b, sb, out, aux, m, n, k,
-                         stream);
-    };
     if (sb_div != 32) {
         // weight scales per row (the reference's packed scale table): the
-        // column-strip kernel
-        int rc = -1;
+        // column-strip kernel only
+        int rc;
         if (M <= 16) {
             const int S = kAccOut ? 1 : strip_splits(M, N, K, wsp.ptr ? wsp.bytes : 0);
             rc = launch_kp<1, 1, 1, 8, BFP4, SMODE, OMODE, 1>(a, sa, b, sb, out, M, N, K, stream, S,
@@ -1235,11 +1230,11 @@ static int gemm_dispatch(const uint8_t *a, const void *sa, const uint8_t *b, con
         // M = 200, N = 8192, K = 1280 24 / 13 (128). bf16
         // results only (the figures are the GEMM's with f32 stores): the f32
         // ones keep the shorter chains.
-        if (M > 64 && exact && OMODE == kOutBf16) {
+        if (M > 64 && math_mode() == WS_MATH_EXACT && !BFP4 && OMODE == kOutBf16) {
             const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
             if (t128 * 4 >= 3l * cu_count() || K <= 2048 ||
                 (K <= 4096 && t128 * 8 >= 3l * cu_count()))
-                rc = tiled();
+                rc = tile_gemm_bf16(SMODE, a, sa, b, sb, out, m, n, k, stream);
         }
         if (rc >= 0) return rc;
         // 5. the other shapes with M > 64: the pipelined split-K kernel

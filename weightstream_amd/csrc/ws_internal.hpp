@@ -46,11 +46,10 @@ int gate_w13_launch(const float *h, const float *gw, float *logits, const uint8_
 int line_gemm(int smode, int omode, const uint8_t *a, const void *sa, const uint8_t *b,
               const void *sb, void *out, int m, int n, int k, hipStream_t stream, int cfg,
               const float *aux = nullptr);
-// gemm_tile.hip: the exact-math FP8 / FP4 GEMM for many rows (whole-K tiles); sbrow: FP8 weight scales per row instead of per 32 rows.
-// -1 when the shape, alignment or output mode does not fit.
-int tile_gemm(bool bfp4, int smode, bool sbrow, int omode, const uint8_t *a, const void *sa,
-              const uint8_t *b, const void *sb, void *out, const float *aux, int64_t m, int64_t n,
-              int64_t k, hipStream_t stream);
+// gemm_tile.hip: the exact-math FP8 GEMM with bf16 results for many rows (whole-K
+// tiles). -1 when the shape or alignment does not fit.
+int tile_gemm_bf16(int smode, const uint8_t *a, const void *sa, const uint8_t *b, const void *sb,
+                   void *out, int64_t m, int64_t n, int64_t k, hipStream_t stream);
 // moe_tile.hip: the grouped gate/up (bf16 h out) and down steps over 96-slot
 // groups, exact math; offsets and counts are the dispatch's. part: scratch of
 // part_bytes for the gate/up sums of the first K part; moe_tile_parts says how
