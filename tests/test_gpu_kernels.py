@@ -673,6 +673,60 @@ def test_tile_gemm_edges_vs_fp64_dequant(m, n, k):
     close(got, da @ (d4 * pw(s4).repeat_interleave(32, 1)).T, "fp4")
 
 
+@pytest.mark.parametrize("split", [True, False])
+@pytest.mark.parametrize("m,n,k", [(130, 272, 768), (130, 272, 896),        # K <= 768 (896): any
+                                   (1030, 4096, 256), (1030, 4112, 256),    # more tiles than CUs
+                                   (380, 400, 1280), (300, 272, 1280),      # 12 and 9 tiles
+                                   (200, 1552, 1536), (150, 1424, 1536),    # 26 and 24
+                                   (200, 2448, 2048), (200, 2320, 2048),    # 40 and 38
+                                   (390, 3984, 2304), (380, 3984, 2304),    # 128 and 96
+                                   (300, 3600, 3200), (300, 5520, 3200),    # 87 and 132
+                                   (600, 4624, 3328),                       # 185
+                                   (380, 4112, 4096), (450, 3088, 4096),    # 99 and 100
+                                   (600, 4880, 4224), (600, 4624, 4224)])   # 195 and 185
+def test_bf16_gemm_each_side_of_the_tile_rule(m, n, k, split):
+    """bf16 results on both sides of each line of the rule that takes them to the whole-K tiles
+    (on the tiles, on the split-K pipeline and without a workspace on its
+    single pass), UE8M0 and f32 scales, against f64; per value the bound of
+    test_tile_gemm_edges_vs_fp64_dequant and one rounding for each of at most 8
+    partial sums."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(m + n + k)
+    announce("bf16 gemm m=%d n=%d k=%d split=%d" % (m, n, k, split))
+    aq = torch.randint(0, 120, (m, k), dtype=torch.uint8, device=DEV, generator=gen)
+    aq |= torch.randint(0, 2, (m, k), dtype=torch.uint8, device=DEV, generator=gen) << 7
+    wq = torch.randint(0, 120, (n, k), dtype=torch.uint8, device=DEV, generator=gen)
+    wq |= torch.randint(0, 2, (n, k), dtype=torch.uint8, device=DEV, generator=gen) << 7
+    sa = torch.randint(118, 126, (m, k // 32), dtype=torch.uint8, device=DEV, generator=gen)
+    sw = torch.randint(110, 118, ((n + 31) // 32, k // 32), dtype=torch.uint8, device=DEV, generator=gen)
+    fa = torch.rand((m, k // 128), device=DEV, generator=gen) + 0.1
+    fw = torch.rand(((n + 127) // 128, k // 128), device=DEV, generator=gen) + 0.1
+    table = torch.from_numpy(O.e4m3_decode_table().astype(np.float64)).to(DEV)
+    pw = lambda s: torch.pow(2.0, s.to(torch.float64) - 127)
+    ca, cw = table[aq.long()], table[wq.long()]
+    ws = torch.empty(L.gemm_workspace_size(m, n, k), dtype=torch.uint8, device=DEV)
+    if split and ws.numel():
+        L.set_gemm_workspace(ws)
+    try:
+        for what in ("ue8m0", "f32s"):
+            out = torch.full((m * n + 64,), -7.0, dtype=torch.bfloat16, device=DEV)
+            if what == "ue8m0":
+                L.fp8_gemm_bf16(aq, sa, wq, sw, out, m, n, k)
+                da = ca * pw(sa).repeat_interleave(32, 1)
+                dw = cw * pw(sw).repeat_interleave(32, 0)[:n].repeat_interleave(32, 1)
+            else:
+                L.fp8_gemm_f32s(aq, fa, wq, fw, out, m, n, k, out_bf16=True)
+                da = ca * fa.double().repeat_interleave(128, 1)
+                dw = cw * fw.double().repeat_interleave(128, 0)[:n].repeat_interleave(128, 1)
+            assert (out[m * n:] == -7).all(), "written past the output"
+            want = da @ dw.T
+            roundings = k // 32 + k // 128 + 2 + 8
+            bound = 2.0 ** -8 * want.abs() + roundings * 2.0 ** -23 * (da.abs() @ dw.abs().T)
+            assert ((out[:m * n].view(m, n).double() - want).abs() <= bound).all(), what
+    finally:
+        L.set_gemm_workspace(None)
+
+
 @pytest.mark.parametrize("m", [65, 130, 520])
 def test_packed_scale_table_above_64_rows(m):
     """ws_fp8_gemm_tl above 64 rows (the column-strip kernel): per-row weight

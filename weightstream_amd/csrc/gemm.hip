@@ -1118,6 +1118,36 @@ static int launch_cfg(const uint8_t *a, const void *sa, const uint8_t *b, const 
     return launch_status();
 }
 
+// Whether the whole-K tiles (gemm_tile.hip) are faster than the kernels they
+// would replace (split-K pipeline, or without a workspace its single pass), by
+// the number t of 128 x 128 tiles. Tiles leave CUs idle where t is small and pay
+// no partials; their time goes in steps of whole rounds. Replaced kernel / tiles,
+// us, cold weights, UE8M0 scales (f32 scales alike but where said):
+//  - K <= 256, more tiles than CUs and none ragged: one or two steps are all
+//    prologue, 777 x 5120 x 128 9.0 / 10.1 (f32 scales 10.3 / 10.0; ragged
+//    3286 x 5216 x 256 29 / 23);
+//  - K <= 768: 1.0-2.9x faster at any t (without a workspace to 896);
+//  - K <= 2048: the line rises with K. K = 1280 t = 8 10.7 / 11.7, 12 12.0 / 11.5,
+//    64 25 / 13; K = 1536 t = 21 13.1 / 13.6, 26 14.5 / 13.9; K = 2048 t = 4 11.4 /
+//    16, 34 15.5 / 16.4, 42 17 / 16.7, 64 25 / 16.5. Without a workspace 36 from
+//    K = 1024 on (t = 30 1.04-1.2x slower, 36 1.5x faster);
+//  - K <= 4096: t = 96 at K = 2304 1.3x, at 4096 0.95x (f32 scales 1.05x), 100 1.0x
+//    (1.1x); between half a round and 0.7 of one the pipeline loses nothing:
+//    t = 132-168 0.91-0.97x above K = 3072 (f32 scales 3584), 180 1.15x (without a
+//    workspace 473 x 4400 x 3712 93 / 34.5);
+//  - above: t = 192 (K = 5120 1.3x), as 160 is 0.88x there. M = N = 4096, K =
+//    8192 372 / 197.
+static bool tiles_pay(int M, int N, int K, bool ue8m0, bool split) {
+    const long t = (long)((M + 127) / 128) * ((N + 127) / 128), cus = cu_count();
+    if (K <= 256 && ue8m0 && N % 128 == 0 && t > cus) return false;
+    if (K <= (split ? 768 : 896)) return true;
+    if (K <= 2048) return t >= (!split ? 36 : K <= 1280 ? 10 : K <= 1536 ? 26 : 40);
+    if (t * 4 >= 3 * cus) return true;
+    if (K > 4096) return false;
+    if (!split || K <= (ue8m0 ? 3072 : 3584)) return t * 8 >= 3 * cus;
+    return t * 10 >= 7 * cus || (t >= (ue8m0 ? 100 : 96) && t * 2 <= cus);
+}
+
 template <bool BFP4, int SMODE, int OMODE>
 // OMODE kOutAcc (C += A.B^T) and kOutAcc2 (C = C + (aux + A.B^T)) run on the
 // kernels with those epilogues (line, column strips), never split over K.
@@ -1220,22 +1250,11 @@ static int gemm_dispatch(const uint8_t *a, const void *sa, const uint8_t *b, con
             if (lc >= 0) rc = line_gemm(SMODE, OMODE, a, sa, b, sb, out, M, N, K, stream, lc, aux);
         }
         if (rc >= 0) return rc;
-        // 4. M > 64, exact math: whole-K tiles (gemm_tile.hip) when they keep
-        // the chip busy: 192 tiles of 128 x 128, 96 at K <= 4096, any number at
-        // K <= 2048 (where the split's partials and their reduction cost more
-        // than the idle CUs). Split-K pipeline against tiles, us: M = 4096,
-        // N = 4096, K = 8192 372 / 197; M = 777, N = 4608, K = 5120 75 / 50 (252
-        // tiles); M = 2000, N = 1280, K = 5120 41 / 47 (160); M = 1024, N =
-        // 2048, K = 4096 33 / 30 (128); M = 200, N = 4096, K = 4096 26 / 29 (64);
-        // M = 200, N = 8192, K = 1280 24 / 13 (128). bf16
-        // results only (the figures are the GEMM's with f32 stores): the f32
-        // ones keep the shorter chains.
-        if (M > 64 && math_mode() == WS_MATH_EXACT && !BFP4 && OMODE == kOutBf16) {
-            const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-            if (t128 * 4 >= 3l * cu_count() || K <= 2048 ||
-                (K <= 4096 && t128 * 8 >= 3l * cu_count()))
-                rc = tile_gemm_bf16(SMODE, a, sa, b, sb, out, m, n, k, stream);
-        }
+        // 4. M > 64, exact math, bf16 results: whole-K tiles where they pay (f32
+        // results keep the shorter chains of the kernels below)
+        if (M > 64 && math_mode() == WS_MATH_EXACT && !BFP4 && OMODE == kOutBf16 &&
+            tiles_pay(M, N, K, SMODE == kUe8m0, wsp.ptr != nullptr))
+            rc = tile_gemm_bf16(SMODE, a, sa, b, sb, out, m, n, k, stream);
         if (rc >= 0) return rc;
         // 5. the other shapes with M > 64: the pipelined split-K kernel
         // (128-row tiles)
