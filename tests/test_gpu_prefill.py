@@ -125,26 +125,28 @@ def _host_experts(slabs, experts, E, dim, inter):
                                                     (40, 256, 640, 384, 6, 10),
                                                     (64, 256, 5120, 2304, 6, 6)])
 def test_moe_prefill_matches_oracle(m, E, dim, inter, k, check):
+    _check_prefill(m, E, dim, inter, k, check)
+
+
+def _check_prefill(m, E, dim, inter, k, check, s=1.1):
+    """ws_moe_prefill against the oracle on `check` rows, popularity Zipf(s);
+    returns the bodies that ran, which must be those the rules name."""
     rng = np.random.default_rng(900 + m + E)
     gen = torch.Generator(device=DEV)
     gen.manual_seed(900 + m)
-    announce("moe_prefill m=%d E=%d dim=%d inter=%d k=%d" % (m, E, dim, inter, k))
+    announce("moe_prefill m=%d E=%d dim=%d inter=%d k=%d s=%.1f" % (m, E, dim, inter, k, s))
     slabs = _slabs(gen, E, dim, inter)
-    logits, bias = zipf_routing(rng, m, E, k)
+    logits, bias = zipf_routing(rng, m, E, k, s)
     idx = torch.empty((m, k), dtype=torch.int32, device=DEV)
     w = torch.empty((m, k), dtype=torch.float32, device=DEV)
     L.moe_topk(dev(logits), dev(bias), None, idx, w, m, E, k, O.SCORE_SIGMOID, 1.0, True, 1.0)
     x = rng.standard_normal((m, dim)).astype(np.float32)
-    ws = torch.empty(L.moe_prefill_workspace_size(m, dim, inter, k, E), dtype=torch.uint8,
-                     device=DEV)
+    ws = _prefill_workspace(m, dim, inter, k, E)
     y = torch.empty((m, dim), dtype=torch.float32, device=DEV)
     L.moe_prefill(dev(x), idx, w, *_packed(slabs, E, dim, inter), y, m, dim, inter, E, k, ws)
-    want_choice = _stationary_expected(idx, E, dim, inter)
-    if want_choice is not None:
-        got = _stationary_choice(ws, m, dim, k, E)
-        print("[moe_prefill m=%d E=%d dim=%d inter=%d] %s bodies" %
-              (m, E, dim, inter, "expert-stationary" if got else "tile-streaming"), flush=True)
-        assert got == want_choice
+    body = _body_ran(ws, m, dim, inter, k, E)
+    print("[moe_prefill m=%d E=%d dim=%d inter=%d] %s bodies" % (m, E, dim, inter, body), flush=True)
+    assert body == _body_expected(idx, E, dim, inter)
     gi, gw, gy = host(idx), host(w), host(y)
     rows = np.linspace(0, m - 1, check).astype(int)
     H = _host_experts(slabs, gi[rows].ravel(), E, dim, inter)
@@ -157,6 +159,7 @@ def test_moe_prefill_matches_oracle(m, E, dim, inter, k, check):
         if staged is None:
             staged = _staged_hidden(x, idx, w, _packed(slabs, E, dim, inter), m, E, dim, inter, k)
         _check_by_stages(gy[r], x[r], gi[r], gw[r], H, staged, r, k, dim, inter)
+    return body
 
 
 @pytest.mark.parametrize("m,E,dim,inter,k", [(120, 16, 768, 384, 4), (200, 32, 2304, 1152, 6),
@@ -166,7 +169,7 @@ def test_moe_prefill_stationary_step_counts(m, E, dim, inter, k):
     """The expert-stationary pair with units of every remainder of four 128-K
     steps (6 and 3, 18 and 9, 10 and 5, 2 and 1, 40 and 19): a unit's repeated
     steps past K multiply nothing. Skewed enough that the dispatch takes it."""
-    test_moe_prefill_matches_oracle(m, E, dim, inter, k, 6)
+    assert _check_prefill(m, E, dim, inter, k, 6) == "stationary"
 
 
 @pytest.mark.parametrize("m,E,dim,inter,k", [(600, 16, 768, 384, 4), (1000, 32, 1280, 640, 4),
@@ -178,7 +181,31 @@ def test_moe_prefill_group_tiles(m, E, dim, inter, k):
     remainder of four (6 and 3, 10 and 5, 4 and 2, 18 and 9, 5 and 1); column
     blocks cut short (inter 384, 640, 1152, 128 of 256; dim 768, 1280, 2304, 640
     of 512)."""
-    test_moe_prefill_matches_oracle(m, E, dim, inter, k, 6)
+    assert _check_prefill(m, E, dim, inter, k, 6) == "groups"
+
+
+@pytest.mark.parametrize("m,E,dim,inter,k,s,body",
+                         [(40, 256, 1792, 384, 8, 0.0, "streaming"),    # K halves of 8 + 6
+                          (40, 256, 2304, 384, 8, 0.0, "stationary"),   # 8 + 10
+                          (40, 256, 4096, 384, 8, 0.0, "streaming"),    # 16 + 16
+                          (40, 256, 4352, 384, 8, 0.0, "stationary"),   # above one pass of A
+                          (40, 256, 2048, 1024, 8, 0.0, "stationary"),  # whole units
+                          (300, 256, 1792, 384, 6, 0.0, "stationary"),  # tiles over 16 rows
+                          (40, 256, 1792, 384, 8, 1.1, None)])          # skewed
+def test_moe_prefill_choice_at_an_even_routing(m, E, dim, inter, k, s, body):
+    """Padded units leave 100 or more short tiles to the tile-streaming pair where
+    its K halves differ little."""
+    got = _check_prefill(m, E, dim, inter, k, 4, s)
+    assert body is None or got == body
+
+
+@pytest.mark.parametrize("m,E,dim,inter,k,body", [(600, 1024, 512, 256, 8, "streaming"),
+                                                  (1024, 1024, 512, 256, 8, "groups"),
+                                                  (96, 16, 384, 256, 4, "streaming")])
+def test_moe_prefill_past_the_stationary_limits(m, E, dim, inter, k, body):
+    """More than 1024 tiles, under and from 8 routes per expert; dim not a multiple
+    of 256."""
+    assert _check_prefill(m, E, dim, inter, k, 4) == body
 
 
 @pytest.mark.parametrize("m,check", [(132, 12), (300, 12), (4500, 8)])
@@ -189,7 +216,7 @@ def test_prefill_all_routes_on_k_experts(m, check):
     the expert-stationary groups (m = 132: 5 tiles per expert, groups of
     2, 2, 1; m = 300: 10 tiles, five full pairs, the last tile 12 rows). At
     m = 4500 the tile capacity exceeds what the stationary bodies take and
-    the tile-streaming pair runs 141 tiles per expert."""
+    the 96-slot groups run 47 of them per expert, the last two strips short."""
     E, dim, inter, k = 64, 2048, 1024, 8
     rng = np.random.default_rng(1700 + m)
     gen = torch.Generator(device=DEV)
@@ -206,17 +233,12 @@ def test_prefill_all_routes_on_k_experts(m, check):
     gi = host(idx)
     assert sorted(set(gi.ravel().tolist())) == sorted(hot.tolist())
     x = rng.standard_normal((m, dim)).astype(np.float32)
-    ws = torch.empty(L.moe_prefill_workspace_size(m, dim, inter, k, E), dtype=torch.uint8,
-                     device=DEV)
+    ws = _prefill_workspace(m, dim, inter, k, E)
     y = torch.empty((m, dim), dtype=torch.float32, device=DEV)
     L.moe_prefill(dev(x), idx, w, *_packed(slabs, E, dim, inter), y, m, dim, inter, E, k, ws)
-    want_choice = _stationary_expected(idx, E, dim, inter)
-    assert want_choice == (1 if m <= 300 else None)
-    if want_choice is not None:
-        got = _stationary_choice(ws, m, dim, k, E)
-        print("[all routes on k experts m=%d] %s bodies" %
-              (m, "expert-stationary" if got else "tile-streaming"), flush=True)
-        assert got == want_choice
+    body = _body_ran(ws, m, dim, inter, k, E)
+    print("[all routes on k experts m=%d] %s bodies" % (m, body), flush=True)
+    assert body == _body_expected(idx, E, dim, inter) == ("stationary" if m <= 300 else "groups")
     gw, gy = host(w), host(y)
     # the first and last rows (first and last tile of every expert) and
     # rows spread between them
@@ -251,33 +273,56 @@ def _a256(v):
     return (v + 255) // 256 * 256
 
 
-def _stationary_expected(idx, E, dim, inter):
-    """The choice the dispatch should make (None where the stationary
-    bodies do not serve the shape): with t_e = ceil(routes of expert e / 32)
-    tiles, nt = sum t_e and ng = sum ceil(t_e / 2) groups, the stationary
-    bodies when 6 (nt - ng) >= nt or nt >= 96."""
+def _body_expected(idx, E, dim, inter):
+    """The bodies ws_moe_prefill should take. From 64 routes per expert on, or
+    from 8 where the capacity is over 1024 tiles, the groups. With t_e = ceil(routes of expert e / 32) tiles, nt =
+    sum t_e and ng = sum ceil(t_e / 2) groups, the stationary pair when 6 (nt
+    - ng) >= nt or nt >= 96; but not on the tile count alone, from 100 tiles, when
+    fewer than 1 in 128 holds over 16 rows, units are padded, dim <= 4096 and the
+    first K half is the longer one and at most 0.6 of the whole."""
     cnt = np.bincount(host(idx).ravel(), minlength=E)
+    routes, tiles = host(idx).size, L.moe_tiles(host(idx).size, E)
+    if routes >= E * (8 if tiles > 1024 else 64):
+        return "groups"
+    if dim % 256 or tiles > 1024:
+        return "streaming"
     t = (cnt + 31) // 32
     nt, ng = int(t.sum()), int(((t + 1) // 2).sum())
-    tiles = L.moe_tiles(host(idx).size, E)
-    fits = (dim % 256 == 0 and (dim // 128) % 8 == 0 and (inter // 128) % 8 == 0 and
-            tiles <= 1024)
-    if not fits:
-        return None
-    return 1 if (6 * (nt - ng) >= nt or nt >= 96) else 0
+    full = int((cnt // 32 + (cnt % 32 > 16)).sum())
+    steps = dim // 128
+    first = (steps + 7) // 8 // 2 * 8
+    balanced = ((steps % 8 or inter // 128 % 8) and dim <= 4096 and 2 * first >= steps
+                and 5 * first <= 3 * steps)
+    if 6 * (nt - ng) >= nt:
+        return "stationary"
+    return "stationary" if nt >= 96 and not (balanced and nt >= 100 and 128 * full < nt) else "streaming"
 
 
-def _stationary_choice(ws, m, dim, k, E):
-    """The body ws_moe_prefill's dispatch chose (1: expert-stationary, 0:
-    tile-streaming), the int32 after the used-tile count in the workspace,
-    whose regions (in order, each 256-byte aligned) are xq, xs, order,
-    layout_w, route_pos, tile_expert, three per-expert arrays, the tile
-    count."""
+_UNTOUCHED = 0x5A
+
+
+def _prefill_workspace(m, dim, inter, k, E):
+    return torch.full((L.moe_prefill_workspace_size(m, dim, inter, k, E),), _UNTOUCHED,
+                      dtype=torch.uint8, device=DEV)
+
+
+def _body_ran(ws, m, dim, inter, k, E):
+    """The bodies that ws_moe_prefill took with a workspace from
+    _prefill_workspace. Its regions (in order, each 256-byte aligned) are xq, xs,
+    order, layout_w, route_pos, tile_expert, three per-expert arrays, the tile count
+    and the dispatch's choice (int32s: 1 stationary, 0 tile-streaming), hq, hs,
+    down, the bf16 tokens and the bf16 h. The groups and the plain tile-streaming
+    pair make no choice; only the groups write the bf16 h."""
     routes = m * k
     slots = L.moe_tiles(routes, E) * 32
     off = (_a256(m * dim) + _a256(m * dim // 32) + 2 * _a256(slots * 4) + _a256(routes * 4) +
            _a256(slots // 32 * 4) + 3 * _a256(E * 4))
-    return int(host(ws[off + 4:off + 8]).view(np.int32)[0])
+    choice = int(host(ws[off + 4:off + 8]).view(np.int32)[0])
+    if choice in (0, 1):
+        return "stationary" if choice else "streaming"
+    assert choice == 0x01010101 * _UNTOUCHED
+    hbf = ws[ws.numel() - _a256(slots * inter * 2):][:slots * inter * 2]
+    return "groups" if bool((hbf != _UNTOUCHED).any()) else "streaming"
 
 
 @pytest.mark.parametrize("zipf", [1.1, 0.275])
@@ -299,15 +344,13 @@ def test_config4_baseline_weights_prefill_matches_oracle(zipf):
     w = torch.empty((m, k), dtype=torch.float32, device=DEV)
     L.moe_topk(dev(logits), dev(bias), None, idx, w, m, E, k, O.SCORE_SIGMOID, 1.0, True, 1.0)
     x = rng.standard_normal((m, dim)).astype(np.float32)
-    ws = torch.empty(L.moe_prefill_workspace_size(m, dim, inter, k, E), dtype=torch.uint8,
-                     device=DEV)
+    ws = _prefill_workspace(m, dim, inter, k, E)
     y = torch.empty((m, dim), dtype=torch.float32, device=DEV)
     P = _packed(slabs, E, dim, inter)
     L.moe_prefill(dev(x), idx, w, *P, y, m, dim, inter, E, k, ws)
     # both draws run the expert-stationary bodies (the skewed one for its
     # shared groups, the mild one for its tile count)
-    assert _stationary_expected(idx, E, dim, inter) == 1
-    assert _stationary_choice(ws, m, dim, k, E) == 1
+    assert _body_ran(ws, m, dim, inter, k, E) == _body_expected(idx, E, dim, inter) == "stationary"
     gi, gw, gy = host(idx), host(w), host(y)
     H = _host_experts(slabs, gi.ravel(), E, dim, inter)
     staged = None
@@ -440,18 +483,33 @@ def test_prefill_stages_compose_to_moe_prefill(m, E, dim, inter, k):
     (which multiplies and writes only the slots that hold routes), on the
     tile-streaming pair and on the bodies that take its place (not on the
     stationary pair's whole units: dim and inter in 1024s)."""
+    y1, y2, _ = _composed(m, E, dim, inter, k)
+    assert np.array_equal(y1.view(np.uint32), y2.view(np.uint32))
+
+
+def _composed(m, E, dim, inter, k, nonfinite=False):
+    """y of ws_moe_prefill, y of its stages, the bodies that ws_moe_prefill took."""
     rng = np.random.default_rng(990 + m)
     gen = torch.Generator(device=DEV)
     gen.manual_seed(990 + m)
-    P = _packed(_slabs(gen, E, dim, inter), E, dim, inter)
+    slabs = _slabs(gen, E, dim, inter)
+    if nonfinite:  # scale bytes of NaN, 2^-127 and 2^127 in one row or another of three experts
+        for j, rows in ((1, inter), (3, inter), (5, dim)):
+            slabs[j].view(E, rows, -1)[0, 3, 1] = 255
+            slabs[j].view(E, rows, -1)[1, 17, 0] = 0
+            slabs[j].view(E, rows, -1)[2, 5, -1] = 254
+    P = _packed(slabs, E, dim, inter)
     logits, bias = zipf_routing(rng, m, E, k)
     idx = torch.empty((m, k), dtype=torch.int32, device=DEV)
     w = torch.empty((m, k), dtype=torch.float32, device=DEV)
     L.moe_topk(dev(logits), dev(bias), None, idx, w, m, E, k, O.SCORE_SIGMOID, 1.0, True, 1.0)
-    x = dev(rng.standard_normal((m, dim)).astype(np.float32))
+    hx = rng.standard_normal((m, dim)).astype(np.float32)
+    if nonfinite:
+        hx[1, 7], hx[2, 40], hx[3, dim - 1] = np.inf, -np.inf, np.nan
+        hx[4], hx[5], hx[6] = np.nan, 3e38, np.float32(1e30) * hx[6]
+    x = dev(hx)
     announce("prefill stages m=%d E=%d dim=%d inter=%d k=%d" % (m, E, dim, inter, k))
-    ws = torch.empty(L.moe_prefill_workspace_size(m, dim, inter, k, E), dtype=torch.uint8,
-                     device=DEV)
+    ws = _prefill_workspace(m, dim, inter, k, E)
     y1 = torch.empty((m, dim), dtype=torch.float32, device=DEV)
     L.moe_prefill(x, idx, w, *P, y1, m, dim, inter, E, k, ws)
 
@@ -471,4 +529,4 @@ def test_prefill_stages_compose_to_moe_prefill(m, E, dim, inter, k):
     L.moe_grouped_down(hq, hs, te, nt, P[4], P[5], down, dim, inter, E, tiles)
     y2 = torch.empty((m, dim), dtype=torch.float32, device=DEV)
     L.moe_combine_f32(down, rp, y2, dim, k, m, tiles)
-    assert np.array_equal(host(y1).view(np.uint32), host(y2).view(np.uint32))
+    return host(y1), host(y2), _body_ran(ws, m, dim, inter, k, E)

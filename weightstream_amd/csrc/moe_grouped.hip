@@ -37,8 +37,15 @@ constexpr int kEsGroup = 2;   // tiles of one expert whose weights the stationar
 // 96 tiles: measured with 384 experts (dim 4096, inter 2048) at M=132 and
 // Zipf(0.25) (237-248 tiles) 620 against 670 us, at M=64 (~140 tiles) 383
 // against 416 us; at M=8 (~51 tiles, one per expert) the two are even.
-__host__ __device__ constexpr bool es_pays(int nt, int ng) {
-    return 6 * (nt - ng) >= nt || nt >= 96;
+// The tile count alone does not pay where `balanced` says that the tile-streaming
+// body has no handicap (padded units against nearly equal K halves in one pass
+// over a tile, see es_balanced) and next to no tile (n16, under 1 in 128) has more than
+// 16 rows, which it multiplies at half the cost. Of 420 calls (70 shapes of 96 to 384
+// experts) that goes for 52, 45 of them 2-17% faster so and none more than 2% slower
+// (3840 x 640, 256 experts, 123 tokens of top-8 250 / 226 us; 4096 x 2304, 66
+// tokens 647 / 590); with 96 to 99 tiles it was up to 18% slower.
+__host__ __device__ constexpr bool es_pays(int nt, int ng, int n16, bool balanced) {
+    return 6 * (nt - ng) >= nt || (nt >= 96 && !(balanced && nt >= 100 && 128 * n16 < nt));
 }
 
 // ---- dispatch (one workgroup) -------------------------------------------
@@ -60,7 +67,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(
     int32_t *__restrict__ offset_out, int32_t *__restrict__ psum_out,
     int32_t *__restrict__ num_tiles_out, int routes, int tiles, int n_experts,
     const float *__restrict__ xf, uint8_t *__restrict__ xq, uint8_t *__restrict__ xs, int64_t nx,
-    uint16_t *__restrict__ xbf, int32_t *__restrict__ select_out) {
+    uint16_t *__restrict__ xbf, int32_t *__restrict__ select_out, int balanced) {
     if (blockIdx.x > 0) {
         // workgroups 1..: the tokens' FP8 1x32 quantisation (the act_quant
         // rule, nx % 32 == 0), independent of the dispatch and run beside it in
@@ -233,7 +240,9 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(
     }
     if (t == 0) *num_tiles_out = used;
     if (select_out) {  // the prefill's choice of body (es_pays over the used tiles)
+        // groups, and above them the tiles of more than 16 rows (at most 1024 of each)
         int g = (padded / kTile + kEsGroup - 1) / kEsGroup;
+        g += (count / kTile + (count % kTile > kTile / 2)) << 16;
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) g += __shfl_xor(g, off, 64);
         if (lane == 0) gsum[w] = g;
@@ -241,7 +250,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(
         if (t == 0) {
             int ng = 0;
             for (int ww = 0; ww < kDispThreads / 64; ww++) ng += gsum[ww];
-            *select_out = es_pays(used, ng) ? 1 : 0;
+            *select_out = es_pays(used, ng & 0xFFFF, ng >> 16, balanced) ? 1 : 0;
         }
     }
     __syncthreads();
@@ -1657,6 +1666,31 @@ static bool es_fits(int64_t dim, int64_t inter, int64_t tiles) {
            tiles <= es::kMaxGroups;
 }
 
+// At most 32 tokens of fewer than 96 routes or experts: one tile per expert and
+// fewer than 96 of them, so es_pays never holds, and the choice on the device
+// (the bf16 tokens, the larger kernels) costs 1-1.5 us (5 tokens of 96 experts,
+// dim 1792, inter 1024, top-4 33.6 / 32.6 us).
+static bool es_never(int64_t rows, int64_t routes, int64_t n_experts) {
+    return rows <= kTile && std::min(routes, n_experts) < 96;
+}
+
+// dim or inter not whole rounds of the ring: padded units.
+static bool es_padded(int64_t dim, int64_t inter) {
+    return dim / 128 % es::kRing || inter / 128 % es::kRing;
+}
+
+// Shapes of padded units that the tile-streaming body serves without a handicap: a
+// tile's A rows staged in one pass (dim <= 4096) and gate/up K halves that
+// differ little, the first being the longer (its waves wait for the longer half: dim
+// 2560, 3072 or 1280 splits 8 + 12, 8 + 16, 8 + 2 steps).
+static bool es_balanced(int64_t dim, int64_t inter) {
+    if (dim > 4096 || !es_padded(dim, inter)) return false;
+    int k0, first;
+    k_part8((int)(dim / 128), 0, 2, k0, first);
+    const int64_t ns = dim / 128;
+    return 2 * first >= ns && 5 * first <= 3 * ns;
+}
+
 // The 96-slot groups of moe_tile.hip: exact math, from 64 routes per expert
 // on, and from 8 where the stationary pair's group table is too small
 // (kMaxGroups tiles). 384 experts, us for the whole prefill, stationary (or, past
@@ -1781,14 +1815,14 @@ static int dispatch_launch(const int32_t *topk_idx, const float *topk_w, int32_t
                            int32_t *num_tiles, int64_t rows, int64_t top_k, int64_t tiles,
                            int64_t n_experts, const float *xf, uint8_t *xq, uint8_t *xs,
                            int64_t nx, ws_stream_t stream, uint16_t *xbf = nullptr,
-                           int32_t *select = nullptr) {
+                           int32_t *select = nullptr, bool balanced = false) {
     const int64_t qblocks = (nx + 4 * kDispThreads - 1) / (4 * kDispThreads);
     const dim3 grid((unsigned)(1 + qblocks));
 #define WS_DISPATCH(M)                                                                         \
     hipLaunchKernelGGL((dispatch_kernel<int32_t, M>), grid, dim3(kDispThreads), 0, stream,     \
                        topk_idx, topk_w, order, layout_w, route_pos, tile_expert, expert_count, \
                        expert_offset, expert_psum, num_tiles, (int)(rows * top_k), (int)tiles,   \
-                       (int)n_experts, xf, xq, xs, nx, xbf, select)
+                       (int)n_experts, xf, xq, xs, nx, xbf, select, (int)balanced)
     if (rows * top_k > kDispHeld * kDispThreads) WS_DISPATCH(true);
     else WS_DISPATCH(false);
 #undef WS_DISPATCH
@@ -1812,7 +1846,7 @@ int ws_moe_dispatch_tl(const int64_t *topk_idx, const float *topk_weights, int32
                        topk_idx, topk_weights, order, layout_weights, route_pos, tile_expert,  \
                        expert_count, expert_offset, expert_psum, num_tiles, (int)(rows * top_k), \
                        (int)tiles, (int)n_experts, nullptr, nullptr, nullptr, (int64_t)0,       \
-                       nullptr, nullptr)
+                       nullptr, nullptr, 0)
     if (many) WS_DISPATCH(true);
     else WS_DISPATCH(false);
 #undef WS_DISPATCH
@@ -2053,10 +2087,11 @@ int ws_moe_prefill(const float *x, const int32_t *topk_idx, const float *topk_w,
     if (n_experts > kMaxExpertsG || routes > (1 << 26) || tiles > (1 << 24)) return WS_ERR_SHAPE;
     const bool tiled = mt_pays(rows, dim, inter, slots, routes, n_experts, tiles) &&
                        moe_tile_parts((size_t)((uint8_t *)xbf - hq), (int)slots, (int)dim, (int)inter) >= 0;
-    const bool stationary = !tiled && es_fits(dim, inter, tiles);
+    const bool stationary = !tiled && es_fits(dim, inter, tiles) && !es_never(rows, routes, n_experts);
     int rc = dispatch_launch(topk_idx, topk_w, order, layout_w, route_pos, tile_expert, cnt, off,
                              psum, ntiles, rows, top_k, tiles, n_experts, x, xq, xs, rows * dim,
-                             stream, stationary || tiled ? xbf : nullptr, stationary ? sel : nullptr);
+                             stream, stationary || tiled ? xbf : nullptr, stationary ? sel : nullptr,
+                             es_balanced(dim, inter));
     if (rc) return rc;
     if (tiled) {
         // its K parts' sums wait in hq .. down, which this step does not use
@@ -2081,8 +2116,7 @@ int ws_moe_prefill(const float *x, const int32_t *topk_idx, const float *topk_w,
         const bool wide = wide_units(tiles);
         const int grows = dim <= 4096 ? 32 : 16;
         const size_t glds = std::max(es::kLdsAll, g_tile_lds(grows, (int)dim));
-        // dim or inter not whole rounds of the ring
-        const bool parts = dim / 128 % es::kRing || inter / 128 % es::kRing;
+        const bool parts = es_padded(dim, inter);
 #define WS_GLU_SEL(R, W, P) \
     hipLaunchKernelGGL((glu_select_kernel<R, W, P>), grid, dim3(kGThreads), glds, stream, sel, ea, ga)
 #define WS_GLU_SEL_P(R, W) { if (parts) WS_GLU_SEL(R, W, true); else WS_GLU_SEL(R, W, false); }

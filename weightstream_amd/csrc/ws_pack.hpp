@@ -68,10 +68,11 @@ __device__ __forceinline__ void fp4_load(Fp4StageU<U> &st, const Fp4Band &b, int
 
 // K range [k0, k1) of part `part` of `parts` over `ksteps` 128-K steps, in
 // whole 8-step stages (so every stage starts on an 8-step scale group).
-__device__ __forceinline__ void k_part8(int ksteps, int part, int parts, int &k0, int &k1) {
+__host__ __device__ __forceinline__ void k_part8(int ksteps, int part, int parts, int &k0, int &k1) {
     const int stages = (ksteps + kU - 1) / kU;
-    k0 = min(ksteps, part * stages / parts * kU);
-    k1 = min(ksteps, (part + 1) * stages / parts * kU);
+    const int a = part * stages / parts * kU, b = (part + 1) * stages / parts * kU;
+    k0 = a < ksteps ? a : ksteps;
+    k1 = b < ksteps ? b : ksteps;
 }
 
 template <int U>
