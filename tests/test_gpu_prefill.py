@@ -176,12 +176,23 @@ def test_moe_prefill_stationary_step_counts(m, E, dim, inter, k):
                                              (4600, 64, 512, 256, 8), (700, 8, 2304, 1152, 2),
                                              (260, 3, 640, 128, 3)])
 def test_moe_prefill_group_tiles(m, E, dim, inter, k):
-    """The 96-slot groups (64 or more routes per expert): experts with no route,
+    """The 96-slot groups (96 or more routes per expert): experts with no route,
     fewer than 32, every strip count and several groups; step counts of every
     remainder of four (6 and 3, 10 and 5, 4 and 2, 18 and 9, 5 and 1); column
     blocks cut short (inter 384, 640, 1152, 128 of 256; dim 768, 1280, 2304, 640
     of 512)."""
     assert _check_prefill(m, E, dim, inter, k, 6) == "groups"
+
+
+@pytest.mark.parametrize("m,E,inter,k", [(512, 128, 2048, 8), (512, 64, 1024, 8),
+                                         (576, 48, 1024, 8)])
+def test_moe_prefill_both_sides_of_the_group_line(m, E, inter, k):
+    """The groups from 32 routes per expert on (four column blocks of 256 or more per
+    CU), 64 (one or more) or 96, and the stationary pair with a token less."""
+    dim = 256
+    assert m * k == E * {2048: 32, 1024: 64 if E == 64 else 96}[inter]
+    assert _check_prefill(m, E, dim, inter, k, 4) == "groups"
+    assert _check_prefill(m - 1, E, dim, inter, k, 4) == "stationary"
 
 
 @pytest.mark.parametrize("m,E,dim,inter,k,s,body",
@@ -274,25 +285,29 @@ def _a256(v):
 
 
 def _body_expected(idx, E, dim, inter):
-    """The bodies ws_moe_prefill should take. From 64 routes per expert on, or
-    from 8 where the capacity is over 1024 tiles, the groups. With t_e = ceil(routes of expert e / 32) tiles, nt =
+    """The bodies ws_moe_prefill should take. From 32, 64 or 96 routes per
+    expert on, by the expert's column blocks, or from 8 where the capacity is
+    over 1024 tiles, the groups. With t_e = ceil(routes of expert e / 32) tiles, nt =
     sum t_e and ng = sum ceil(t_e / 2) groups, the stationary pair when 6 (nt
     - ng) >= nt or nt >= 96; but not on the tile count alone, from 100 tiles, when
     fewer than 1 in 128 holds over 16 rows, units are padded, dim <= 4096 and the
     first K half is the longer one and at most 0.6 of the whole."""
     cnt = np.bincount(host(idx).ravel(), minlength=E)
     routes, tiles = host(idx).size, L.moe_tiles(host(idx).size, E)
-    if routes >= E * (8 if tiles > 1024 else 64):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    blocks = E * ((inter + 255) // 256)
+    steps = dim // 128
+    padded = bool(steps % 8 or inter // 128 % 8)
+    per = 32 if blocks >= (4 if padded else 8) * cus else 64 if blocks >= cus else 96
+    if routes >= E * (8 if tiles > 1024 else per):
         return "groups"
     if dim % 256 or tiles > 1024:
         return "streaming"
     t = (cnt + 31) // 32
     nt, ng = int(t.sum()), int(((t + 1) // 2).sum())
     full = int((cnt // 32 + (cnt % 32 > 16)).sum())
-    steps = dim // 128
     first = (steps + 7) // 8 // 2 * 8
-    balanced = ((steps % 8 or inter // 128 % 8) and dim <= 4096 and 2 * first >= steps
-                and 5 * first <= 3 * steps)
+    balanced = padded and dim <= 4096 and 2 * first >= steps and 5 * first <= 3 * steps
     if 6 * (nt - ng) >= nt:
         return "stationary"
     return "stationary" if nt >= 96 and not (balanced and nt >= 100 and 128 * full < nt) else "streaming"

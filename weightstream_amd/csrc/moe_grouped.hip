@@ -1691,19 +1691,31 @@ static bool es_balanced(int64_t dim, int64_t inter) {
     return 2 * first >= ns && 5 * first <= 3 * ns;
 }
 
-// The 96-slot groups of moe_tile.hip: exact math, from 64 routes per expert
-// on, and from 8 where the stationary pair's group table is too small
-// (kMaxGroups tiles). 384 experts, us for the whole prefill, stationary (or, past
-// 1024 tiles, tile-streaming) pair / groups: dim 4096, inter 2048, top-8 at
-// 12.5 / 32 / 42 routes per expert 889 / 985, 1406 / 1355, 1600 / 1520; 62 and
-// 85 (streaming) 2556 / 1414, 3816 / 2191; dim 5120, inter 2304, top-6 at 62
-// (streaming) 5814 / 2437; 96 experts, dim 2304, inter 1152 at 125 420 / 380.
+// The 96-slot groups of moe_tile.hip: exact math, from as many routes per expert
+// on as make them faster than the pair below. Whole prefill, us, stationary (or, past
+// its table of kMaxGroups tiles, tile-streaming) pair / groups, popularity even
+// and Zipf(0.6):
+//  - 384 experts, dim 4096, inter 2048, top-8: 24 routes per expert 1077 / 1152 and
+//    1244 / 1221, 32 1237 / 1237 and 1419 / 1388, 48 1547 / 1423 and 1759 /
+//    1662; dim 5120, inter 2304, top-6: 24 1629 / 1651 and 1815 / 1785, 32 1837 /
+//    1766 and 2078 / 1977, 48 2291 / 2020 and 2649 / 2386;
+//  - fewer column blocks than 4 per CU (E experts x inter / 256; 8 against whole
+//    units, which are faster: 256 experts, 3072 x 1024, top-4, 34 379 / 368 and 444 / 459)
+//    leave CUs without a unit: 96 experts, dim 2304, inter 1152, top-6 (480 blocks): 48 217 / 183
+//    and 215 / 226, 64 247 / 207 and 254 / 247; below one block per CU, 64 experts,
+//    dim 1024, inter 512, top-4: 64 75 / 79 and 76 / 83, 96 92 / 89 and 90 / 90;
+//  - past the table, from 8: 1024 experts, dim 2048, inter 1024, top-8: 6 713 / 744
+//    and 538 / 435, 8 751 / 754 and 644 / 538; 384 experts, dim 4096, 56 (the
+//    fewest there) 2547 / 1555 and 2659 / 1820.
 // The sums, and so the bits, are the tile-streaming pair's.
 static bool mt_pays(int64_t rows, int64_t dim, int64_t inter, int64_t slots, int64_t routes,
                     int64_t n_experts, int64_t tiles) {
     if (math_mode() != WS_MATH_EXACT) return false;
     if (rows * dim * 2 >= (1ll << 32) || slots * inter * 2 >= (1ll << 32)) return false;  // 32-bit rows
-    return routes >= 64 * n_experts || (tiles > es::kMaxGroups && routes >= 8 * n_experts);
+    if (tiles > es::kMaxGroups) return routes >= 8 * n_experts;
+    const int64_t blocks = n_experts * ((inter + 255) / 256), cus = cu_count();
+    const int64_t many = (es_padded(dim, inter) ? 4 : 8) * cus;
+    return routes >= (blocks >= many ? 32 : blocks >= cus ? 64 : 96) * n_experts;
 }
 
 // ---- combine: y[row] = sum of its routes' outputs in ascending slot order --
