@@ -545,3 +545,19 @@ def _composed(m, E, dim, inter, k, nonfinite=False):
     y2 = torch.empty((m, dim), dtype=torch.float32, device=DEV)
     L.moe_combine_f32(down, rp, y2, dim, k, m, tiles)
     return host(y1), host(y2), _body_ran(ws, m, dim, inter, k, E)
+
+
+@pytest.mark.parametrize("m,E,dim,inter,k,body", [(200, 32, 2304, 1152, 6, "stationary"),
+                                                  (130, 8, 256, 128, 2, "stationary"),
+                                                  (1000, 32, 1280, 640, 4, "groups"),
+                                                  (700, 8, 2304, 1152, 2, "groups"),
+                                                  (9, 16, 512, 256, 4, "streaming")])
+def test_prefill_nonfinite_tokens_and_weights_compose(m, E, dim, inter, k, body):
+    """Infinities, NaN and values near the type's largest in tokens, NaN and
+    extreme weight scales: the same rows are NaN and the others have the same bits on
+    every body."""
+    y1, y2, ran = _composed(m, E, dim, inter, k, nonfinite=True)
+    assert ran == body
+    nan = np.isnan(y1)
+    assert nan.any() and not nan.all() and np.array_equal(nan, np.isnan(y2))
+    assert np.array_equal(y1[~nan].view(np.uint32), y2[~nan].view(np.uint32))
