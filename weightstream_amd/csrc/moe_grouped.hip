@@ -58,6 +58,12 @@ __device__ __forceinline__ int id_of(int64_t v, int n_experts) {
     return v >= 0 && v < n_experts ? (int)v : -1;
 }
 
+// Values per lane of the dispatch's quantisation workgroups. With few routes one:
+// four leave the launch's first workgroup, which is its length, waiting for more of
+// the others' code and loads (27 tokens of 384 experts, dim 4096 7.3 us with four
+// and 6.6 with one, 512 18.3 and 17.5).
+__host__ __device__ constexpr int disp_quant_per_lane(bool many) { return many ? 4 : 1; }
+
 // MANY: more routes than the kDispHeld chunks held in registers.
 template <typename IdxT, bool MANY>
 __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(
@@ -69,13 +75,14 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(
     const float *__restrict__ xf, uint8_t *__restrict__ xq, uint8_t *__restrict__ xs, int64_t nx,
     uint16_t *__restrict__ xbf, int32_t *__restrict__ select_out, int balanced) {
     if (blockIdx.x > 0) {
+        constexpr int kQ = disp_quant_per_lane(MANY);
         // workgroups 1..: the tokens' FP8 1x32 quantisation (the act_quant
         // rule, nx % 32 == 0), independent of the dispatch and run beside it in
         // the same launch; with xbf also the exact bf16 of each quantised value
-        // (byte times block scale). Four values per lane, a block being 8 lanes,
-        // when xf is 16-byte aligned (one 4-byte store per lane, not one byte), else one
-        // and a half-wave.
-        if (((uintptr_t)xf & 15) == 0) {
+        // (byte times block scale). Many routes: four values per lane, a block being 8
+        // lanes, when xf is 16-byte aligned (one 4-byte store per lane, not one
+        // byte). Otherwise one and a half-wave.
+        if (MANY && ((uintptr_t)xf & 15) == 0) {
             const int64_t i = ((int64_t)(blockIdx.x - 1) * kDispThreads + threadIdx.x) * 4;
             const bool live = i < nx;
             uint32_t sb;
@@ -92,7 +99,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(
             }
             return;
         }
-        for (int64_t i = (int64_t)(blockIdx.x - 1) * kDispThreads * 4 + threadIdx.x, k = 0; k < 4;
+        for (int64_t i = (int64_t)(blockIdx.x - 1) * kDispThreads * kQ + threadIdx.x, k = 0; k < kQ;
              k++, i += kDispThreads) {
             const bool live = i < nx;
             uint32_t sb;
@@ -1320,18 +1327,20 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
     // of the stream (real == false) the last step's loads are repeated and
     // not used, so that every step has the same loads in flight after it.
     auto issue = [&](EsStep &x, int slot, bool real) {
-        const int sl = PAD ? min(s_i, NS - 1) : s_i;
+        // a function, not a value: its multiples held in registers cost the units
+        // without padding 0.6 us (down, 27 tokens)
+        auto sl = [&]() { return (uint32_t)(PAD ? min(s_i, NS - 1) : s_i); };
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const int m = MODE == 0 ? h : 0;
             x.q[h] = __builtin_bit_cast(
-                u32x4v, __builtin_amdgcn_raw_buffer_load_b128(wr[m], bo[h] + (uint32_t)sl * 1024u, 0, 0));
+                u32x4v, __builtin_amdgcn_raw_buffer_load_b128(wr[m], bo[h] + sl() * 1024u, 0, 0));
         }
         const uint32_t lb = ring + slot * kSlotB + 4 * w * kRowB;
 #pragma unroll
         for (int j = 0; j < kTG; j++)
             if ((cmask >> j) & 1)  // uniform: tiles the group has, rows with routes
-                es_dma(abuf, ao[j] + (uint32_t)sl * kRowB, lb + j * kTile * kRowB, 16);
+                es_dma(abuf, ao[j] + sl() * kRowB, lb + j * kTile * kRowB, 16);
         nT[slot] = __builtin_popcount(cmask);
         if (real && ++s_i == NSP) {
             s_i = 0;
@@ -1350,13 +1359,12 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
     // is held over the stream is spilled beside p0, and a reload from scratch
     // waits for every load in flight
     auto lane_at_use = [&]() {
-        int l = lane;
-        if (kParts)
-            __asm__ volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
+        int l;
+        __asm__ volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
         return l;
     };
     auto open_compute = [&]() {
-        const int r = lane_at_use() & 15;
+        const int ru = kParts ? lane_at_use() & 15 : r;
         const int k = unit_k(ri_c);
         const int v = __builtin_amdgcn_readfirstlane(es_lds_word(&grp_l[k / NCG]));
         nrc = __builtin_amdgcn_readfirstlane(es_lds_word(&nrl_l[k / NCG]));
@@ -1374,7 +1382,7 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
 #pragma unroll
                 for (int i = 0; i < 2; i++)
                     rwf[j][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                        lwbuf, (uint32_t)(slot0 + 16 * i + r) * 4u, 0, 0));
+                        lwbuf, (uint32_t)(slot0 + 16 * i + ru) * 4u, 0, 0));
             }
     };
     // [tile][band][16-row fragment]: the weights are the MFMA's first
@@ -1485,8 +1493,8 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
         // columns; a row's FP8 1x32 block spans this wave (lanes g = 0..3 of
         // the row's r) and its partner (w ^ 1), which meet in LDS (both
         // tiles' maxima across one barrier)
-        const int ln = lane_at_use(), r = ln & 15, g = ln >> 4;
-        const int col = (kParts ? unit_k(ri_c) % NCG : cgc) * 128 + 16 * w + 4 * g;
+        const int ln = kParts ? lane_at_use() : lane, ru = kParts ? ln & 15 : r, gu = kParts ? ln >> 4 : g;
+        const int col = (kParts ? unit_k(ri_c) % NCG : cgc) * 128 + 16 * w + 4 * gu;
         if (kParts) {
 #pragma unroll
             for (int j = 0; j < kTG; j++)
@@ -1505,7 +1513,7 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
             const int nr = (nrc >> (8 * j)) & 0xFF;
 #pragma unroll
             for (int i = 0; i < 2; i++) {
-                const int row = 16 * i + r;
+                const int row = 16 * i + ru;
                 const float rw = rwf[j][i];
                 m[j][i] = 0.0f;
 #pragma unroll
@@ -1528,9 +1536,9 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
             }
         }
         // the row maxima of the wave's 16 columns: am_l[w][j * 32 + row]
-        const uint32_t base = lds_addr(&am_l[0][0]) + (uint32_t)r * 4u;
+        const uint32_t base = lds_addr(&am_l[0][0]) + (uint32_t)ru * 4u;
         static_assert(kTG == 2, "two tiles per group");
-        if (g == 0) {
+        if (gu == 0) {
             es_lds_put2(base + (uint32_t)w * kTG * kTile * 4u, m[0][0], m[0][1]);
             es_lds_put2(base + (uint32_t)(w * kTG + 1) * kTile * 4u, m[1][0], m[1][1]);
         }
@@ -1544,7 +1552,7 @@ __device__ __forceinline__ void es_body(const EsArgs &a, uint8_t *g_lds) {
             const int slot0 = min(t0c + j, a.slots / kTile - 1) * kTile;
 #pragma unroll
             for (int i = 0; i < 2; i++) {
-                const int row = 16 * i + r;
+                const int row = 16 * i + ru;
                 // the rule of quant_fp8_block32 on the 1x32 block
                 float mm = fmaxf(m[j][i], mp[j][i]);
                 if (!(mm >= 1e-4f)) mm = 1e-4f;
@@ -1828,14 +1836,15 @@ static int dispatch_launch(const int32_t *topk_idx, const float *topk_w, int32_t
                            int64_t n_experts, const float *xf, uint8_t *xq, uint8_t *xs,
                            int64_t nx, ws_stream_t stream, uint16_t *xbf = nullptr,
                            int32_t *select = nullptr, bool balanced = false) {
-    const int64_t qblocks = (nx + 4 * kDispThreads - 1) / (4 * kDispThreads);
-    const dim3 grid((unsigned)(1 + qblocks));
+    const bool many = rows * top_k > kDispHeld * kDispThreads;
+    const int64_t per = kDispThreads * disp_quant_per_lane(many);
+    const dim3 grid((unsigned)(1 + (nx + per - 1) / per));
 #define WS_DISPATCH(M)                                                                         \
     hipLaunchKernelGGL((dispatch_kernel<int32_t, M>), grid, dim3(kDispThreads), 0, stream,     \
                        topk_idx, topk_w, order, layout_w, route_pos, tile_expert, expert_count, \
                        expert_offset, expert_psum, num_tiles, (int)(rows * top_k), (int)tiles,   \
                        (int)n_experts, xf, xq, xs, nx, xbf, select, (int)balanced)
-    if (rows * top_k > kDispHeld * kDispThreads) WS_DISPATCH(true);
+    if (many) WS_DISPATCH(true);
     else WS_DISPATCH(false);
 #undef WS_DISPATCH
     return launch_status();
