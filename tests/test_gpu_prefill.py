@@ -78,6 +78,55 @@ def test_dispatch_bit_exact(m, E, k):
                           want["layout_w"][:used].view(np.uint32))
 
 
+@pytest.mark.parametrize("m,E,k", [(512, 384, 8), (513, 384, 8), (4097, 5, 1), (900, 1024, 16)])
+def test_dispatch_with_dropped_ids_around_4096_routes(m, E, k):
+    """Both rankings (routes held in registers up to 4096, a run of routes per
+    wave above) with ids another rank owns and one popular expert."""
+    rng = np.random.default_rng(820 + m)
+    idx = np.stack([rng.choice(E, k, replace=False) for _ in range(m)]).astype(np.int32)
+    idx[rng.random((m, k)) < 0.2] = -1
+    idx[m // 3: m // 2, 0] = 2
+    idx[-1] = -1
+    w = rng.random((m, k)).astype(np.float32)
+    tiles = L.moe_tiles(m * k, E)
+    announce("moe_dispatch with dropped ids m=%d E=%d k=%d" % (m, E, k))
+    got, want = _dispatch_gpu(idx, w, E, tiles), O.dispatch(idx, w, E, tiles)
+    used = want["num_tiles"] * 32
+    assert got["num_tiles"][0] == want["num_tiles"]
+    for key in ("route_pos", "tile_expert", "count", "offset", "psum"):
+        assert np.array_equal(got[key], want[key]), key
+    for key in ("order", "layout_w"):
+        assert np.array_equal(got[key][:used].view(np.uint32), want[key][:used].view(np.uint32)), key
+
+
+@pytest.mark.parametrize("rows", [2047, 2048])   # one row per add; groups of 4, 6 or 8
+@pytest.mark.parametrize("top_k", [1, 3, 4, 5, 6, 7, 8, 9, 16])
+def test_combine_adds_in_slot_order(rows, top_k):
+    """The ordered sum of a row's slots, dropped ones left out, whole and ragged
+    groups of loads: the bits of the same f32 adds, infinities and NaN among them."""
+    dim, tiles = 132, 64
+    rng = np.random.default_rng(830 + top_k)
+    down = rng.standard_normal((tiles * 32, dim)).astype(np.float32)
+    down[5, 3], down[9, 4], down[11, 5] = np.inf, -np.inf, np.nan
+    pos = np.stack([rng.choice(tiles * 32, top_k, replace=False) for _ in range(rows)]).astype(np.int32)
+    pos[rng.random(pos.shape) < 0.1] = -1
+    pos[1] = -1
+    out = torch.full((rows * dim + 64,), -7.0, device=DEV)
+    announce("combine rows=%d top_k=%d" % (rows, top_k))
+    L.moe_combine_f32(dev(down), dev(pos), out, dim, top_k, rows, tiles)
+    want = np.zeros((rows, dim), np.float32)
+    padded = np.concatenate([down, np.zeros((1, dim), np.float32)])
+    order = np.sort(np.where(pos < 0, tiles * 32, pos), axis=1)
+    for j in range(top_k):
+        # a dropped slot adds nothing: the sum stays (+0 for a row of none)
+        want = np.where((order[:, j] < tiles * 32)[:, None], want + padded[order[:, j]], want)
+    got = host(out)
+    assert (got[rows * dim:] == -7).all()
+    got, nan = got[:rows * dim].reshape(rows, dim), np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
+
+
 def _slabs(gen, E, dim, inter):
     """Raw (on-disk layout) expert slabs; the kernels read _packed(raw)."""
     w1, s1 = rand_fp4_weights(gen, E * inter, dim)
