@@ -247,6 +247,7 @@ def test_moe_prefill_both_sides_of_the_group_line(m, E, inter, k):
 @pytest.mark.parametrize("m,E,dim,inter,k,s,body",
                          [(40, 256, 1792, 384, 8, 0.0, "streaming"),    # K halves of 8 + 6
                           (40, 256, 2304, 384, 8, 0.0, "stationary"),   # 8 + 10
+                          (40, 256, 3328, 384, 8, 0.0, "streaming"),    # 16 + 10
                           (40, 256, 4096, 384, 8, 0.0, "streaming"),    # 16 + 16
                           (40, 256, 4352, 384, 8, 0.0, "stationary"),   # above one pass of A
                           (40, 256, 2048, 1024, 8, 0.0, "stationary"),  # whole units
@@ -340,7 +341,7 @@ def _body_expected(idx, E, dim, inter):
     sum t_e and ng = sum ceil(t_e / 2) groups, the stationary pair when 6 (nt
     - ng) >= nt or nt >= 96; but not on the tile count alone, from 100 tiles, when
     fewer than 1 in 128 holds over 16 rows, units are padded, dim <= 4096 and the
-    first K half is the longer one and at most 0.6 of the whole."""
+    first K half is the longer one and at most 8 / 13 of the whole."""
     cnt = np.bincount(host(idx).ravel(), minlength=E)
     routes, tiles = host(idx).size, L.moe_tiles(host(idx).size, E)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
@@ -356,7 +357,7 @@ def _body_expected(idx, E, dim, inter):
     nt, ng = int(t.sum()), int(((t + 1) // 2).sum())
     full = int((cnt // 32 + (cnt % 32 > 16)).sum())
     first = (steps + 7) // 8 // 2 * 8
-    balanced = padded and dim <= 4096 and 2 * first >= steps and 5 * first <= 3 * steps
+    balanced = padded and dim <= 4096 and 2 * first >= steps and 13 * first <= 8 * steps
     if 6 * (nt - ng) >= nt:
         return "stationary"
     return "stationary" if nt >= 96 and not (balanced and nt >= 100 and 128 * full < nt) else "streaming"

@@ -35,9 +35,10 @@ __global__ __launch_bounds__(256) void act_quant_kernel(float *xio, const float 
 
 // Four values per lane and kAqPasses x 4 KB of f32 per workgroup (the loads of
 // all passes are issued first), a block being 8 lanes: one float4 load and one
-// 4-byte store per lane where the kernel above moves a float and a byte, so
-// that the kernel is bound by HBM and not by its memory instructions. 33.5 M
-// values (M = 4096, K = 8192): 105 -> 44 us (3.8 TB/s). Same bytes; taken when the
+// 4-byte store per lane where the kernel above moves a float and a byte. What
+// bounds it is the vector ALU (the bytes' rounding; 94% of its cycles), no longer the
+// memory instructions. 33.5 M values (M = 4096, K = 8192): 105 -> 44 us (3.8
+// TB/s). Same bytes; taken when the
 // operands are aligned for it (x 16 bytes, q 4).
 constexpr int kAqPasses = 2;
 template <int MODE>  // 0: emit bytes, 1: snap in place

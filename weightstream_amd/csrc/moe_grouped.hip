@@ -1690,13 +1690,14 @@ static bool es_padded(int64_t dim, int64_t inter) {
 // Shapes of padded units that the tile-streaming body serves without a handicap: a
 // tile's A rows staged in one pass (dim <= 4096) and gate/up K halves that
 // differ little, the first being the longer (its waves wait for the longer half: dim
-// 2560, 3072 or 1280 splits 8 + 12, 8 + 16, 8 + 2 steps).
+// 2560, 3072 or 1280 splits 8 + 12, 8 + 16, 8 + 2 steps; 3328, the most uneven that is
+// taken, 16 + 10).
 static bool es_balanced(int64_t dim, int64_t inter) {
     if (dim > 4096 || !es_padded(dim, inter)) return false;
     int k0, first;
     k_part8((int)(dim / 128), 0, 2, k0, first);
     const int64_t ns = dim / 128;
-    return 2 * first >= ns && 5 * first <= 3 * ns;
+    return 2 * first >= ns && 13 * first <= 8 * ns;
 }
 
 // The 96-slot groups of moe_tile.hip: exact math, from as many routes per expert

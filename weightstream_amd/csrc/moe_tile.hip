@@ -28,7 +28,8 @@
 //    the outputs' 2-norm error against 64 bits 9.3e-5 and 8.0e-5 for two draws,
 //    6.6e-5 and 4.7e-5 so). The registers hold one sum (192 of 256 would go to
 //    two), so p0 waits in scratch memory, 192 KB per workgroup that its next unit
-//    takes again: 2099 -> 2159 us for that prefill.
+//    takes again (6 MB per XCD: they leave its L2, 0.54 GB written): 2099 -> 2159
+//    us for that prefill.
 // The strips (16 rows) multiplied are those that hold routes: six
 // instantiations, 16 to 96 rows.
 #include "ws_internal.hpp"
@@ -424,8 +425,8 @@ __global__ __launch_bounds__(kThreads) void moe_tile_kernel(const Args p) {
 
 }  // namespace mt
 
-// 0: no scratch needed (one K part), 1: a slice per workgroup (the slices stay
-// in the caches), 2: where those do not fit (few slots), a piece per strip and
+// 0: no scratch needed (one K part), 1: a slice per workgroup (48 MB, taken again
+// by its next unit), 2: where those do not fit (few slots), a piece per strip and
 // 32 columns; -1: neither fits.
 int moe_tile_parts(size_t part_bytes, int slots, int dim, int inter) {
     if ((dim / 128 + kU - 1) / kU < 2) return 0;
