@@ -113,9 +113,11 @@ int ws_weight_quant_fp8(const float *w, uint8_t *q, uint8_t *s, int64_t rows, in
  * (device, stream): GEMMs issued on `stream` (NULL = the default stream) of
  * the current device use the workspace registered for that stream, so GEMMs
  * on different streams never share one. With a workspace, GEMMs with M > 64
- * and few tiles (and M <= 16 with few column strips and K > 8192) split K across
- * workgroups and a second kernel adds the f32 partials in split order
- * (deterministic); without one they use the single-pass kernels. Calls on one
+ * that no whole-K kernel serves (f32 results at any number of tiles; bf16
+ * results with few 128 x 128 tiles for their K), and those with M <= 16, few
+ * column strips and K > 8192, split K across workgroups and a second kernel
+ * adds the f32 partials in split order (deterministic); without one they use
+ * the single-pass kernels. bf16 results of many tiles need none. Calls on one
  * stream are ordered by the stream, so they may share its workspace.
  * ws_gemm_workspace_size gives the bytes a shape needs; a smaller workspace
  * makes that shape use the single-pass kernel. Workspace NULL unregisters the
